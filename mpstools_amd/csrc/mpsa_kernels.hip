@@ -72,6 +72,68 @@ __device__ __forceinline__ int find_task(const Task* tasks, int ntasks, int t, i
   return lo;
 }
 
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+// The same search by all 64 lanes of a wave at once (every lane active, t
+// uniform): a round reads 64 tasks' numbers, so 64 tasks take one memory
+// latency and 4096 two, where the binary search takes 6 and 12 one after
+// another.  Short tiles spend a good part of their time here.
+template <typename Task>
+__device__ __forceinline__ int find_task_wave(const Task* tasks, int ntasks, int t, int Task::*field) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0, n = ntasks;  // the task lies in [lo, lo + n)
+  while (n > 1) {
+    const int step = (n + 63) >> 6;
+    const int i = lane * step;
+    const bool ok = i < n && tasks[lo + (i < n ? i : 0)].*field <= t;
+    const int c = __popcll(__ballot(ok)) - 1;
+    lo += c * step;
+    n = min(step, n - c * step);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// A workgroup's copy of the tasks' first tiles: the search then costs LDS
+// latencies (64 tasks a round) where it would wait for memory two or three
+// times per tile.  Lists longer than kMaxKeys are searched in memory.  Only
+// the wave tiles use it (t-V D = 512, 64 vectors, stage 1: 197 us against
+// 217); the workgroup tiles lose more to the 8 KB of LDS (235 against 295).
+constexpr int kMaxKeys = 2048;
+__device__ __forceinline__ void load_keys(int* keys, const GTask* __restrict__ tasks, int ntasks) {
+  if (ntasks > kMaxKeys) return;
+  for (int i = threadIdx.x; i < ntasks; i += blockDim.x) keys[i] = tasks[i].tile0;
+  __syncthreads();
+}
+__device__ __forceinline__ int find_key(const int* keys, int n, int t) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0;
+  while (n > 1) {
+    const int step = (n + 63) >> 6;
+    const int i = lane * step;
+    const bool ok = i < n && keys[lo + (i < n ? i : 0)] <= t;
+    const int c = __popcll(__ballot(ok)) - 1;
+    lo += c * step;
+    n = min(step, n - c * step);
+  }
+  return uni(lo);
+}
+
+// The task owning t, given the one (ti >= 0) of a smaller or equal number
+// served just before, or ti = -1.  Workers take runs of consecutive numbers,
+// so most steps cost one scalar read instead of a search.
+template <typename Task>
+__device__ __forceinline__ int next_task(const Task* tasks, int ntasks, int t, int Task::*field, int ti) {
+  if (ti < 0 || tasks[ti].*field > t) return find_task_wave(tasks, ntasks, t, field);
+  while (ti + 1 < ntasks && tasks[ti + 1].*field <= t) ++ti;
+  return uni(ti);
+}
+// Length of those runs: workers still take turns at least eight times over a
+// launch, since the tasks come longest first.  Lists searched in LDS need none.
+__device__ __forceinline__ int run_length(int total, int workers, bool keyed) {
+  if (keyed) return 1;
+  const int r = total / (8 * workers);
+  return r < 1 ? 1 : (r > 8 ? 8 : r);
+}
+
 // Position of a k-step iterator over the segments of one task, with the
 // segment's descriptor held in registers: memory is read only when the
 // iterator enters a new segment, never per k-step.
@@ -80,7 +142,6 @@ struct SegCursor {
   int64_t a_off, b_off;
   double alpha;
 };
-__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 // Plans never emit segments with k <= 0, so entering a segment is one uniform
 // (scalar) descriptor read.
 __device__ __forceinline__ void cur_enter(SegCursor& c, const GSeg* __restrict__ segs, int si, int send) {
@@ -123,224 +184,488 @@ __device__ __forceinline__ __hip_bfloat16 cvt<__hip_bfloat16, double>(double x) 
   return __float2bfloat16((float)x);
 }
 
+// Workgroup barrier for data exchanged through LDS only: waits for this wave's
+// LDS accesses and not, as __syncthreads does, for its global loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Where a folded operand's major index (a column of op(B) or a row of op(A)
+// counted over all vectors) lies: vector v, index r inside its block.
+struct FoldPos {
+  int v, r;
+};
+// The quotient is below 4096 (the vector count of a folded launch), so the
+// single-precision estimate is off by one at most.
+__device__ __forceinline__ FoldPos fold_pos(int i, int n) {
+  FoldPos p;
+  p.v = (int)((float)i * __builtin_amdgcn_rcpf((float)n));
+  p.r = i - p.v * n;
+  if (p.r < 0) {
+    p.v -= 1;
+    p.r += n;
+  } else if (p.r >= n) {
+    p.v += 1;
+    p.r -= n;
+  }
+  return p;
+}
+
+// Batched launches (nvec > 1) whose A (FOLD 1) or B (FOLD 2) is shared by all
+// vectors treat the vectors' blocks as one matrix: columns (v, j) of op(B) and
+// C, or rows (v, i) of op(A) and C, so a block dimension is padded to the tile
+// once per task and not once per vector, and the shared operand is read once
+// per tile of several vectors.  Tiles keep the per-vector numbering of the
+// plan: a task owns nvec * (its tiles) slots, and the slots beyond its folded
+// tile count are empty.
+template <int FOLD>
+struct TilePos {
+  int ti, v, tm, tn;
+  bool ok;
+};
+template <int FOLD, int BM, int BN>
+__device__ __forceinline__ TilePos<FOLD> tile_pos(const GTask* __restrict__ tasks, int ntasks, int g,
+                                                  int tiles_per_vec, int nvec, const int* keys, int prev) {
+  TilePos<FOLD> p;
+  p.v = FOLD == 0 ? g / tiles_per_vec : 0;
+  const int t = FOLD == 0 ? g - p.v * tiles_per_vec : g / nvec;
+  p.ti = keys && ntasks <= kMaxKeys ? find_key(keys, ntasks, t) : next_task(tasks, ntasks, t, &GTask::tile0, prev);
+  const GTask& tk = tasks[p.ti];
+  const int local = FOLD == 0 ? t - tk.tile0 : g - tk.tile0 * nvec;
+  const int tiles_m = FOLD == 2 ? (tk.m * nvec + BM - 1) / BM : tk.tiles_m;
+  p.tm = local % tiles_m;
+  p.tn = local / tiles_m;
+  p.ok = FOLD == 0 || p.tn < (FOLD == 1 ? (tk.n * nvec + BN - 1) / BN : (tk.n + BN - 1) / BN);
+  return p;
+}
+
 // ---------------------------------------------------------------------------
-// FP64 / FP32 grouped GEMM, 16x16x4 MFMA.  256 threads = 4 waves in 2x2; each
-// wave owns a (BM/2)x(BN/2) sub-tile.  A and B tiles go through LDS (k-major);
-// the next k-step's global loads are issued into registers before the MFMAs of
-// the current step.
+// FP64 / FP32 grouped GEMM, 16x16x4 MFMA.  256 threads = 4 waves over a BM x BN
+// tile.  A and B slabs of BK k-steps go through two LDS buffers (k-major), so
+// a slab costs one barrier; the next slab's global loads are issued into
+// registers before the MFMAs of the current one.  Row pitch BM + 4: the four
+// k-groups of a fragment read and the transposing writes both fall on distinct
+// banks.  A thread keeps a pointer to each of its rows for a segment; k is
+// clamped to the segment and masked on its last slab, and rows past the block
+// are clamped to its last row (their results are never stored).
+// k order (all FP64/FP32 kernels of this file, so that results do not depend
+// on the tile class): chunks of 16 from a segment's start, MFMA q of a chunk
+// takes k = 4 * (lane / 16) + q.
 // ---------------------------------------------------------------------------
-template <typename T, typename TOut, int BM, int BN, bool TA, bool TB>
+// Loads of one operand of a workgroup tile: a slab of BK k-steps of BR rows,
+// NV values per thread.  KC: k contiguous (thread: k fixed, rows IR apart),
+// else rows contiguous (thread: row fixed, k-steps KR apart).
+template <typename T, int BR, int BK, bool KC, bool FOLD>
+struct SlabOperand {
+  static constexpr int NV = BR * BK / 256;
+  static constexpr int NR = KC ? NV : 1;
+  static constexpr int IR = 256 / BK, KR = KC ? 1 : 256 / BR;
+  int row[NR];                // inside its vector's block, clamped
+  int64_t vo[FOLD ? NR : 1];  // its vector's offset
+  const T* p[NR];             // its first element in the segment
+  static __device__ __forceinline__ int k_of(int r) {
+    const int tid = threadIdx.x;
+    return KC ? tid % BK : tid / BR + r * KR;
+  }
+  static __device__ __forceinline__ int row_of(int r) {
+    const int tid = threadIdx.x;
+    return KC ? tid / BK + r * IR : tid % BR;
+  }
+  __device__ __forceinline__ void init(int first, int len, int block, int64_t vs) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      int x = min(first + row_of(r), len - 1);
+      if (FOLD) {
+        const FoldPos q = fold_pos(x, block);
+        x = q.r;
+        vo[FOLD ? r : 0] = (int64_t)q.v * vs;
+      }
+      row[r] = x;
+    }
+  }
+  __device__ __forceinline__ void enter(const T* base, int ld) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      p[r] = base + (FOLD ? vo[FOLD ? r : 0] : 0) + (KC ? (int64_t)row[r] * ld : (int64_t)row[r]);
+  }
+  // k-steps kk .. kk + BK - 1 of the segment, of which rem exist
+  __device__ __forceinline__ void load(T (&x)[NV], int kk, int rem, int ld) const {
+    if (KC) {
+      const int kc = kk + min(k_of(0), rem - 1);
+#pragma unroll
+      for (int r = 0; r < NV; ++r) x[r] = p[KC ? r : 0][kc];
+    } else {
+      const T* b = p[0] + (int64_t)kk * ld;
+#pragma unroll
+      for (int r = 0; r < NV; ++r) x[r] = b[(int64_t)min(k_of(r), rem - 1) * ld];
+    }
+  }
+};
+
+template <typename T, typename TOut, int BM, int BN, bool TA, bool TB, int FOLD>
 __global__ __launch_bounds__(256, 2) void gemm16_kernel(const GTask* __restrict__ tasks, int ntasks,
                                                         const GSeg* __restrict__ segs, int tiles_per_vec,
-                                                        int total_tiles, const T* __restrict__ A, int64_t a_vs,
-                                                        const T* __restrict__ B, int64_t b_vs,
+                                                        int total_tiles, int nvec, const T* __restrict__ A,
+                                                        int64_t a_vs, const T* __restrict__ B, int64_t b_vs,
                                                         TOut* __restrict__ C, int64_t c_vs) {
-  constexpr int BK = 16;
-  constexpr int PA = BM + 2, PB = BN + 2;
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
-  constexpr int NA = BM * BK / 256, NB = BN * BK / 256;
+  // 128-byte k-slabs per row for the 128x128 tile in both types
+  constexpr int BK = (sizeof(T) == 4 && BM == 128 && BN == 128) ? 32 : 16;
+  constexpr int PA = BM + 4, PB = BN + 4;
+  constexpr int TM = BM / 32, TN = BN / 32;  // 16x16 sub-tiles of a wave (2 x 2 waves)
+  typedef SlabOperand<T, BM, BK, TA, FOLD == 2> OpA;
+  typedef SlabOperand<T, BN, BK, !TB, FOLD == 1> OpB;
+  constexpr int NA = OpA::NV, NB = OpB::NV;
   typedef typename Acc4<T>::type V4;
-  __shared__ T As[BK][PA];
-  __shared__ T Bs[BK][PB];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ T As[2][BK][PA];
+  __shared__ T Bs[2][BK][PB];
+  const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   const int l16 = lane & 15, lq = lane >> 4;
 
-  for (int g = xcd_logical_id(); g < total_tiles; g += gridDim.x) {
-    const int v = g / tiles_per_vec;
-    const int t = g - v * tiles_per_vec;
-    const int ti_ = find_task(tasks, ntasks, t, &GTask::tile0);
-    const GTask tk = tasks[ti_];
-    const int local = t - tk.tile0;
-    const int tm = local % tk.tiles_m, tn = local / tk.tiles_m;
-    const int row0 = tm * BM, col0 = tn * BN;
-    const int m = tk.m, n = tk.n;
+  const int run = run_length(total_tiles, gridDim.x, false);
+  for (int g0 = xcd_logical_id() * run, i0 = 0, ti = -1; g0 < total_tiles;) {
+    const int g = g0 + i0;
+    if (++i0 == run || g + 1 >= total_tiles) {  // the run's last tile
+      i0 = 0;
+      g0 += gridDim.x * run;
+    }
+    const TilePos<FOLD> tp = tile_pos<FOLD, BM, BN>(tasks, ntasks, g, tiles_per_vec, nvec, nullptr, ti);
+    ti = i0 == 0 ? -1 : tp.ti;
+    if (!tp.ok) continue;
+    const GTask tk = tasks[tp.ti];
+    const int row0 = tp.tm * BM, col0 = tp.tn * BN;
+    const int m = uni(tk.m), n = uni(tk.n);
+    const int mf = FOLD == 2 ? m * nvec : m, nf = FOLD == 1 ? n * nvec : n;
+    const int wr0 = row0 + wm * TM * 16, wc0 = col0 + wn * TN * 16;
     V4 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = V4{0, 0, 0, 0};
 
+    const T* Av = A + (FOLD == 0 ? (int64_t)tp.v * a_vs : 0);
+    const T* Bv = B + (FOLD == 0 ? (int64_t)tp.v * b_vs : 0);
+    OpA oa;
+    OpB ob;
+    oa.init(row0, mf, m, a_vs);
+    ob.init(col0, nf, n, b_vs);
     const int send = tk.seg0 + tk.nseg;
-    SegCursor cl;  // position of the step held in registers
-    cur_enter(cl, segs, tk.seg0, send);
+    SegCursor cl;  // position of the slab held in registers
     T ra[NA], rb[NB];
-    unsigned oka = 0, okb = 0;  // in-bounds flags, applied at the LDS store so loads stay in flight
     T ralpha = (T)1;
-    auto load = [&](const SegCursor& c) {
-      const T* Ab = A + (int64_t)v * a_vs + c.a_off;
-      const T* Bb = B + (int64_t)v * b_vs + c.b_off;
-      ralpha = (T)c.alpha;
-      const int kk0 = c.kk;
-      oka = 0;
-      okb = 0;
-#pragma unroll
-      for (int r = 0; r < NA; ++r) {
-        const int e = tid + r * 256;
-        int i, kk;
-        if (!TA) { i = e % BM; kk = e / BM; }
-        else { kk = e % BK; i = e / BK; }
-        const int gi = row0 + i, gk = kk0 + kk;
-        const bool ok = gi < m && gk < c.k;
-        const int gic = gi < m ? gi : m - 1, gkc = gk < c.k ? gk : c.k - 1;  // always-valid address
-        ra[r] = TA ? Ab[gkc + (int64_t)gic * c.lda] : Ab[gic + (int64_t)gkc * c.lda];
-        oka |= (ok ? 1u : 0u) << r;
-      }
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        const int e = tid + r * 256;
-        int j, kk;
-        if (!TB) { kk = e % BK; j = e / BK; }
-        else { j = e % BN; kk = e / BN; }
-        const int gj = col0 + j, gk = kk0 + kk;
-        const bool ok = gj < n && gk < c.k;
-        const int gjc = gj < n ? gj : n - 1, gkc = gk < c.k ? gk : c.k - 1;
-        rb[r] = TB ? Bb[gjc + (int64_t)gkc * c.ldb] : Bb[gkc + (int64_t)gjc * c.ldb];
-        okb |= (ok ? 1u : 0u) << r;
+    int rk = 0;  // k-steps of the slab held in registers
+    auto enter = [&](int si) {
+      cur_enter(cl, segs, si, send);
+      if (si < send) {
+        oa.enter(Av + cl.a_off, cl.lda);
+        ob.enter(Bv + cl.b_off, cl.ldb);
       }
     };
-    auto store = [&]() {
-#pragma unroll
-      for (int r = 0; r < NA; ++r) {
-        const int e = tid + r * 256;
-        int i, kk;
-        if (!TA) { i = e % BM; kk = e / BM; }
-        else { kk = e % BK; i = e / BK; }
-        As[kk][i] = ((oka >> r) & 1u) ? ra[r] * ralpha : (T)0;
-      }
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        const int e = tid + r * 256;
-        int j, kk;
-        if (!TB) { kk = e % BK; j = e / BK; }
-        else { j = e % BN; kk = e / BN; }
-        Bs[kk][j] = ((okb >> r) & 1u) ? rb[r] : (T)0;
-      }
+    auto load = [&]() {
+      rk = uni(cl.k - cl.kk);
+      ralpha = (T)cl.alpha;
+      oa.load(ra, cl.kk, rk, cl.lda);
+      ob.load(rb, cl.kk, rk, cl.ldb);
     };
-    if (cl.si < send) load(cl);
+    auto store = [&](int b) {
+      if (ralpha != (T)1) {
+#pragma unroll
+        for (int r = 0; r < NA; ++r) ra[r] *= ralpha;
+      }
+      if (rk < BK) {
+#pragma unroll
+        for (int r = 0; r < NA; ++r)
+          if (OpA::k_of(r) >= rk) ra[r] = (T)0;
+#pragma unroll
+        for (int r = 0; r < NB; ++r)
+          if (OpB::k_of(r) >= rk) rb[r] = (T)0;
+      }
+#pragma unroll
+      for (int r = 0; r < NA; ++r) As[b][OpA::k_of(r)][OpA::row_of(r)] = ra[r];
+#pragma unroll
+      for (int r = 0; r < NB; ++r) Bs[b][OpB::k_of(r)][OpB::row_of(r)] = rb[r];
+    };
+    int buf = 0;
+    enter(tk.seg0);
+    if (cl.si < send) load();
     while (cl.si < send) {
-      __syncthreads();  // previous MFMAs done reading LDS
-      store();
-      __syncthreads();
-      cur_next(cl, segs, send, BK);
-      if (cl.si < send) load(cl);
+      // buffer `buf` was last read two slabs ago, before every wave passed
+      // the previous slab's barrier
+      store(buf);
+      const int kn = uni(rk);  // k-steps of this slab
+      lds_barrier();
+      cl.kk += BK;
+      if (cl.kk >= cl.k) enter(uni(cl.si) + 1);
+      if (cl.si < send) load();
+      const T* as = &As[buf][4 * lq][wm * TM * 16 + l16];
+      const T* bs = &Bs[buf][4 * lq][wn * TN * 16 + l16];
 #pragma unroll
       for (int kq = 0; kq < BK / 4; ++kq) {
+        const int kr = (kq / 4) * 16 + kq % 4;
+        if (kr >= kn) continue;  // uniform
         T af[TM], bf[TN];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) af[i] = As[kq * 4 + lq][wm * WM + i * 16 + l16];
+        for (int i = 0; i < TM; ++i) af[i] = as[kr * PA + i * 16];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) bf[j] = Bs[kq * 4 + lq][wn * WN + j * 16 + l16];
+        for (int j = 0; j < TN; ++j) bf[j] = bs[kr * PB + j * 16];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(af[i], bf[j], acc[i][j]);
       }
+      buf ^= 1;
     }
     // epilogue: see acc_row for the row each accumulator register holds
-    TOut* Cb = C + (int64_t)v * c_vs + tk.c_off;
+    TOut* Cb = C + (FOLD == 0 ? (int64_t)tp.v * c_vs : 0) + tk.c_off;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int col = col0 + wn * WN + j * 16 + l16;
+      for (int r = 0; r < 4; ++r) {
+        const int row = wr0 + i * 16 + acc_row<T>(lq, r);
+        if (row >= mf) continue;
+        int64_t ro = row;
+        if (FOLD == 2) {
+          const FoldPos p = fold_pos(row, m);
+          ro = (int64_t)p.v * c_vs + p.r;
+        }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = row0 + wm * WM + i * 16 + acc_row<T>(lq, r);
-          if (row < m && col < n) Cb[row + (int64_t)col * m] = cvt<TOut>(acc[i][j][r]);
+        for (int j = 0; j < TN; ++j) {
+          const int col = wc0 + j * 16 + l16;
+          if (col >= nf) continue;
+          int64_t co = (int64_t)col * m;
+          if (FOLD == 1) {
+            const FoldPos p = fold_pos(col, n);
+            co = (int64_t)p.v * c_vs + (int64_t)p.r * m;
+          }
+          Cb[ro + co] = cvt<TOut>(acc[i][j][r]);
         }
       }
-    __syncthreads();
+    lds_barrier();  // the next tile's first slab may go to a buffer still being read
   }
 }
 
 // ---------------------------------------------------------------------------
 // FP64 / FP32 grouped GEMM for small sector blocks: one WTxWT output tile per
 // wave (WT = 16 or 32: 1 or 2x2 16x16x4 MFMA tiles), four independent waves
-// per workgroup, no LDS and no barrier.  Each MFMA takes its A fragment
-// (lane: row l16, k lq) and B fragment (k lq, column l16) straight from
-// global memory (the blocks of a small sector stay in L1/L2); four k-steps of
-// loads are issued ahead of their MFMAs, and a 32-wide tile reuses each
-// fragment for two MFMAs.  Tiles are numbered as for gemm16_kernel
-// (m-fastest inside a task) and every output element is accumulated over k
-// in the same order, so FP64 results equal gemm16_kernel's bit for bit;
-// loads clamp to valid addresses and zero what lies outside the block.
+// per workgroup and no barrier.  The loads of the next chunks of 16 k, across
+// segment boundaries, are in flight while a chunk's MFMAs run: a tile's k
+// loop is a serial chain of L2 latencies otherwise.  An operand
+// whose rows are contiguous is loaded as its MFMA fragments (16 rows x 4 k, a
+// 128-byte line per k in FP64); one whose k are contiguous is loaded along k
+// (16 k of 4 rows) and transposed through the wave's own LDS, since as
+// fragments it would touch 16 lines per load.  Sub-tiles of a 32-wide tile
+// that lie outside the block are not multiplied.  Tiles are numbered and
+// every output element is accumulated over k as in gemm16_kernel, so FP64
+// results equal its bit for bit; loads clamp to valid addresses.
 // ---------------------------------------------------------------------------
-template <typename T, typename TOut, bool TA, bool TB, int WT>
+// Loads of one operand of a wave tile: NT sub-tiles of 16 rows, four values
+// per lane and sub-tile of a chunk of 16 k.  KC: k contiguous.
+template <typename T, int NT, bool KC, bool FOLD>
+struct WaveOperand {
+  static constexpr int NR = KC ? 4 : 1;           // rows per lane and sub-tile
+  static constexpr int P = sizeof(T) == 8 ? 18 : 20;  // LDS row pitch: 16-byte reads on distinct banks
+  int row[NT][NR];                                // inside its vector's block, clamped
+  int64_t vo[FOLD ? NT : 1][FOLD ? NR : 1];       // its vector's offset
+  __device__ __forceinline__ void init(int first, int len, int block, int64_t vs) {
+    const int l16 = threadIdx.x & 15, lq = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        int x = min(first + 16 * i + (KC ? 4 * r + lq : l16), len - 1);
+        if (FOLD) {
+          const FoldPos p = fold_pos(x, block);
+          x = p.r;
+          vo[FOLD ? i : 0][FOLD ? r : 0] = (int64_t)p.v * vs;
+        }
+        row[i][r] = x;
+      }
+  }
+  // base: the segment's operand advanced to the chunk's first k; rem: its k-steps
+  __device__ __forceinline__ void load(T (&x)[NT][4], const T* __restrict__ base, int ld, int rem) const {
+    const int l16 = threadIdx.x & 15, lq = (threadIdx.x & 63) >> 4;
+    if (KC) {
+      const int kc = min(l16, rem - 1);
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int q = KC ? r : 0;
+          x[i][r] = base[(FOLD ? vo[FOLD ? i : 0][FOLD ? q : 0] : 0) + (int64_t)row[i][q] * ld + kc];
+        }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const unsigned ko = __umul24(min(4 * lq + q, rem - 1), ld);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) x[i][q] = (base + (FOLD ? vo[FOLD ? i : 0][0] : 0) + row[i][0])[ko];
+      }
+    }
+  }
+  // x as MFMA fragments: x[i][q] at row l16, k = 4 lq + q
+  static __device__ __forceinline__ void fragments(T (&x)[NT][4], T* __restrict__ lds) {
+    if (!KC) return;
+    const int l16 = threadIdx.x & 15, lq = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lds[(16 * i + 4 * r + lq) * P + l16] = x[i][r];
+    // a wave's LDS accesses execute in program order; this keeps the compiler's
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      typedef T V4 __attribute__((ext_vector_type(4)));
+      const V4 v = *reinterpret_cast<const V4*>(lds + (16 * i + l16) * P + 4 * lq);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[i][q] = v[q];
+    }
+    asm volatile("" ::: "memory");
+  }
+};
+
+template <typename T, typename TOut, bool TA, bool TB, int WT, int FOLD>
 __global__ __launch_bounds__(256) void gemm_wave_kernel(const GTask* __restrict__ tasks, int ntasks,
                                                         const GSeg* __restrict__ segs, int tiles_per_vec,
-                                                        int total_tiles, const T* __restrict__ A, int64_t a_vs,
-                                                        const T* __restrict__ B, int64_t b_vs,
+                                                        int total_tiles, int nvec, const T* __restrict__ A,
+                                                        int64_t a_vs, const T* __restrict__ B, int64_t b_vs,
                                                         TOut* __restrict__ C, int64_t c_vs) {
   typedef typename Acc4<T>::type V4;
   constexpr int NT = WT / 16;
+  typedef WaveOperand<T, NT, TA, FOLD == 2> OpA;
+  typedef WaveOperand<T, NT, !TB, FOLD == 1> OpB;
+  constexpr int LA = TA ? WT * OpA::P : 0, LB = TB ? 0 : WT * OpB::P;
+  __shared__ __attribute__((aligned(32))) T lds[4][LA + LB > 0 ? LA + LB : 4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, lq = lane >> 4;
   const int nw = gridDim.x * 4;
-  for (int g = xcd_logical_id() * 4 + wave; g < total_tiles; g += nw) {
-    const int v = g / tiles_per_vec;
-    const int t = g - v * tiles_per_vec;
-    const GTask tk = tasks[find_task(tasks, ntasks, t, &GTask::tile0)];
-    const int local = t - tk.tile0;
-    const int row0 = (local % tk.tiles_m) * WT, col0 = (local / tk.tiles_m) * WT;
-    const int m = tk.m, n = tk.n;
-    bool rok[NT], cok[NT];
-    int rowc[NT], colc[NT];  // always-valid addresses
-#pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const int row = row0 + 16 * i + l16, col = col0 + 16 * i + l16;
-      rok[i] = row < m;
-      cok[i] = col < n;
-      rowc[i] = rok[i] ? row : m - 1;
-      colc[i] = cok[i] ? col : n - 1;
+  __shared__ int keys[kMaxKeys];
+  load_keys(keys, tasks, ntasks);
+  const int run = run_length(total_tiles, nw, ntasks <= kMaxKeys);
+  for (int g0 = uni(xcd_logical_id() * 4 + wave) * run, i0 = 0, ti = -1; g0 < total_tiles;) {
+    const int g = g0 + i0;
+    if (++i0 == run || g + 1 >= total_tiles) {  // the run's last tile
+      i0 = 0;
+      g0 += nw * run;
     }
+    const TilePos<FOLD> tp = tile_pos<FOLD, WT, WT>(tasks, ntasks, g, tiles_per_vec, nvec, keys, ti);
+    ti = i0 == 0 ? -1 : tp.ti;
+    if (!tp.ok) continue;
+    const GTask tk = tasks[tp.ti];
+    const int row0 = tp.tm * WT, col0 = tp.tn * WT;
+    const int m = uni(tk.m), n = uni(tk.n);
+    const int mf = FOLD == 2 ? m * nvec : m, nf = FOLD == 1 ? n * nvec : n;
+    const int ntm = uni(min(NT, (mf - row0 + 15) >> 4)), ntn = uni(min(NT, (nf - col0 + 15) >> 4));
+    OpA oa;
+    OpB ob;
+    oa.init(row0, mf, m, a_vs);
+    ob.init(col0, nf, n, b_vs);
+    const T* Av = A + (FOLD == 0 ? (int64_t)tp.v * a_vs : 0);
+    const T* Bv = B + (FOLD == 0 ? (int64_t)tp.v * b_vs : 0);
     V4 acc[NT][NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[i][j] = V4{0, 0, 0, 0};
     const int send = tk.seg0 + tk.nseg;
-    for (int si = tk.seg0; si < send; ++si) {
-      const GSeg sg = segs[uni(si)];
-      const int k = uni(sg.k), lda = uni(sg.lda), ldb = uni(sg.ldb);
-      const T* Ab = A + (int64_t)v * a_vs + sg.a_off;
-      const T* Bb = B + (int64_t)v * b_vs + sg.b_off;
-      const T alpha = (T)sg.alpha;
-      for (int k0 = 0; k0 < k; k0 += 16) {
-        T af[4][NT], bf[4][NT];
+
+    struct Chunk {
+      T a[NT][4], b[NT][4];
+      T alpha;
+      int k;  // k-steps of the chunk (uniform)
+    };
+    SegCursor cl;
+    cur_enter(cl, segs, tk.seg0, send);
+    bool ended = tk.nseg == 0;
+    // k is clamped here and masked when the chunk is multiplied
+    auto load = [&](Chunk& c) {
+      const int rem = uni(cl.k - cl.kk);
+      c.k = rem;
+      c.alpha = (T)cl.alpha;
+      oa.load(c.a, Av + cl.a_off + (TA ? (int64_t)cl.kk : (int64_t)cl.kk * cl.lda), cl.lda, rem);
+      ob.load(c.b, Bv + cl.b_off + (TB ? (int64_t)cl.kk * cl.ldb : (int64_t)cl.kk), cl.ldb, rem);
+      if (cl.kk + 16 < cl.k) cl.kk += 16;
+      else if (uni(cl.si) + 1 < send) cur_enter(cl, segs, uni(cl.si) + 1, send);
+      else ended = true;
+    };
+    auto compute = [&](Chunk& c) {
+      // every load of the chunk is waited for here, also those that the
+      // branches below leave unused: one still in flight would hold up the
+      // next use of its register with a wait for all loads
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int kk = k0 + 4 * q + lq;
-          const bool kok = kk < k;
-          const int kc = kok ? kk : k - 1;
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-          for (int i = 0; i < NT; ++i) {
-            const T a = TA ? Ab[kc + (int64_t)rowc[i] * lda] : Ab[rowc[i] + (int64_t)kc * lda];
-            const T b = TB ? Bb[colc[i] + (int64_t)kc * ldb] : Bb[kc + (int64_t)colc[i] * ldb];
-            af[q][i] = (rok[i] && kok) ? a * alpha : (T)0;
-            bf[q][i] = (cok[i] && kok) ? b : (T)0;
-          }
-        }
+        for (int i = 0; i < NT; ++i) asm volatile("" : "+v"(c.a[i][q]), "+v"(c.b[i][q]));
+      OpA::fragments(c.a, lds[wave]);
+      OpB::fragments(c.b, lds[wave] + LA);
+      if (c.k < 16) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          if (k0 + 4 * q < k)  // uniform: k0, q and k are the same in every lane
+          if (4 * lq + q >= c.k) {
 #pragma unroll
-            for (int i = 0; i < NT; ++i)
+            for (int i = 0; i < NT; ++i) {
+              c.a[i][q] = (T)0;
+              c.b[i][q] = (T)0;
+            }
+          }
+      }
 #pragma unroll
-              for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(af[q][i], bf[q][j], acc[i][j]);
+      for (int q = 0; q < 4; ++q) {
+        if (q >= c.k) break;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          if (i >= ntm) break;
+          const T a = c.a[i][q] * c.alpha;
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            if (j < ntn) acc[i][j] = mfma16(a, c.b[j][q], acc[i][j]);
+        }
+      }
+    };
+    // The next chunk's loads are in flight behind the computed one.  No load is
+    // conditional inside an iteration: the compiler can then wait for a chunk
+    // by count, not for all loads in flight.
+    if (!ended) {
+      Chunk x, y;
+      load(x);
+      while (true) {
+        if (ended) {
+          compute(x);
+          break;
+        }
+        load(y);
+        compute(x);
+        if (ended) {
+          compute(y);
+          break;
+        }
+        load(x);
+        compute(y);
       }
     }
-    TOut* Cb = C + (int64_t)v * c_vs + tk.c_off;
+    TOut* Cb = C + (FOLD == 0 ? (int64_t)tp.v * c_vs : 0) + tk.c_off;
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int orow = row0 + 16 * i + acc_row<T>(lq, r);
-          const int ocol = col0 + 16 * j + l16;
-          if (orow < m && ocol < n) Cb[orow + (int64_t)ocol * m] = cvt<TOut>(acc[i][j][r]);
+      for (int r = 0; r < 4; ++r) {
+        const int row = row0 + 16 * i + acc_row<T>(lq, r);
+        if (row >= mf) continue;
+        int64_t ro = row;
+        if (FOLD == 2) {
+          const FoldPos p = fold_pos(row, m);
+          ro = (int64_t)p.v * c_vs + p.r;
         }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const int col = col0 + 16 * j + l16;
+          if (col >= nf) continue;
+          int64_t co = (int64_t)col * m;
+          if (FOLD == 1) {
+            const FoldPos p = fold_pos(col, n);
+            co = (int64_t)p.v * c_vs + (int64_t)p.r * m;
+          }
+          Cb[ro + co] = cvt<TOut>(acc[i][j][r]);
+        }
+      }
   }
 }
 
@@ -407,7 +732,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(const GTask* __restri
   for (int g = xcd_logical_id(); g < total_tiles; g += gridDim.x) {
     const int v = g / tiles_per_vec;
     const int t = g - v * tiles_per_vec;
-    const GTask tk = tasks[find_task(tasks, ntasks, t, &GTask::tile0)];
+    const GTask tk = tasks[find_task_wave(tasks, ntasks, t, &GTask::tile0)];
     const int local = t - tk.tile0;
     const int tm = local % tk.tiles_m, tn = local / tk.tiles_m;
     const int row0 = tm * BM, col0 = tn * BN;
@@ -1628,10 +1953,13 @@ __global__ __launch_bounds__(256) void mix_kernel(const MixTask* __restrict__ ta
                                                   const MixTerm* __restrict__ terms, int chunks_per_vec,
                                                   int total_chunks, const T* __restrict__ src, T* __restrict__ dst,
                                                   int64_t vs) {
-  for (int g = blockIdx.x; g < total_chunks; g += gridDim.x) {
+  const int run = (total_chunks + gridDim.x - 1) / gridDim.x;  // consecutive chunks per workgroup
+  const int gend = min(total_chunks, (int)(blockIdx.x + 1) * run);
+  for (int g = blockIdx.x * run, ti = -1; g < gend; ++g) {
     const int v = g / chunks_per_vec;
     const int c = g - v * chunks_per_vec;
-    const MixTask tk = tasks[find_task(tasks, ntasks, c, &MixTask::chunk0)];
+    ti = next_task(tasks, ntasks, c, &MixTask::chunk0, ti);
+    const MixTask tk = tasks[ti];
     const int64_t base = (int64_t)(c - tk.chunk0) * 1024;
     const T* sv = src + (int64_t)v * vs;
     T* dv = dst + (int64_t)v * vs + tk.dst_off;
@@ -1655,10 +1983,13 @@ __global__ __launch_bounds__(256) void mix_kernel<double, double>(const MixTask*
                                                                   int chunks_per_vec, int total_chunks,
                                                                   const double* __restrict__ src,
                                                                   double* __restrict__ dst, int64_t vs) {
-  for (int g = blockIdx.x; g < total_chunks; g += gridDim.x) {
+  const int run = (total_chunks + gridDim.x - 1) / gridDim.x;  // consecutive chunks per workgroup
+  const int gend = min(total_chunks, (int)(blockIdx.x + 1) * run);
+  for (int g = blockIdx.x * run, ti = -1; g < gend; ++g) {
     const int v = g / chunks_per_vec;
     const int c = g - v * chunks_per_vec;
-    const MixTask tk = tasks[find_task(tasks, ntasks, c, &MixTask::chunk0)];
+    ti = next_task(tasks, ntasks, c, &MixTask::chunk0, ti);
+    const MixTask tk = tasks[ti];
     const int64_t base = (int64_t)(c - tk.chunk0) * 1024;
     const double* sv = src + (int64_t)v * vs;
     double* dv = dst + (int64_t)v * vs + tk.dst_off;
@@ -1691,10 +2022,13 @@ __global__ __launch_bounds__(128) void mix_bf16_kernel(const MixTask* __restrict
                                                        __hip_bfloat16* __restrict__ dst, int64_t vs, int64_t plane) {
   const unsigned short* su = reinterpret_cast<const unsigned short*>(src);
   unsigned short* du = reinterpret_cast<unsigned short*>(dst);
-  for (int g = blockIdx.x; g < total_chunks; g += gridDim.x) {
+  const int run = (total_chunks + gridDim.x - 1) / gridDim.x;  // consecutive chunks per workgroup
+  const int gend = min(total_chunks, (int)(blockIdx.x + 1) * run);
+  for (int g = blockIdx.x * run, ti = -1; g < gend; ++g) {
     const int v = g / chunks_per_vec;
     const int c = g - v * chunks_per_vec;
-    const MixTask tk = tasks[find_task(tasks, ntasks, c, &MixTask::chunk0)];
+    ti = next_task(tasks, ntasks, c, &MixTask::chunk0, ti);
+    const MixTask tk = tasks[ti];
     const int64_t e = (int64_t)(c - tk.chunk0) * 1024 + threadIdx.x * 8;
     if (e >= tk.len) continue;
     const unsigned short* sv = su + (int64_t)v * vs;
@@ -2114,10 +2448,13 @@ template <typename TO>
 __global__ __launch_bounds__(256) void repack_kernel(const Repack* __restrict__ tasks, int ntasks, int chunks_per_vec,
                                                      int total, const double* __restrict__ src, int64_t s_vs,
                                                      TO* __restrict__ dst, int64_t d_vs) {
-  for (int g = blockIdx.x; g < total; g += gridDim.x) {
+  const int run = (total + gridDim.x - 1) / gridDim.x;  // consecutive chunks per workgroup
+  const int gend = min(total, (int)(blockIdx.x + 1) * run);
+  for (int g = blockIdx.x * run, ti = -1; g < gend; ++g) {
     const int v = g / chunks_per_vec;
     const int c = g - v * chunks_per_vec;
-    const Repack tk = tasks[find_task(tasks, ntasks, c, &Repack::chunk0)];
+    ti = next_task(tasks, ntasks, c, &Repack::chunk0, ti);
+    const Repack tk = tasks[ti];
     const int64_t len = (int64_t)tk.rows * tk.cols;
     const int64_t base = (int64_t)(c - tk.chunk0) * 1024;
     const double* s = src + (int64_t)v * s_vs + tk.src_off;
@@ -2141,10 +2478,13 @@ __global__ __launch_bounds__(256) void repack_split_kernel(const Repack* __restr
                                                            int chunks_per_vec, int total, const double* __restrict__ src,
                                                            int64_t s_vs, __hip_bfloat16* __restrict__ dst,
                                                            int64_t d_vs, int64_t plane) {
-  for (int g = blockIdx.x; g < total; g += gridDim.x) {
+  const int run = (total + gridDim.x - 1) / gridDim.x;  // consecutive chunks per workgroup
+  const int gend = min(total, (int)(blockIdx.x + 1) * run);
+  for (int g = blockIdx.x * run, ti = -1; g < gend; ++g) {
     const int v = g / chunks_per_vec;
     const int c = g - v * chunks_per_vec;
-    const Repack tk = tasks[find_task(tasks, ntasks, c, &Repack::chunk0)];
+    ti = next_task(tasks, ntasks, c, &Repack::chunk0, ti);
+    const Repack tk = tasks[ti];
     const int64_t len = (int64_t)tk.rows * tk.cols;
     const int64_t base = (int64_t)(c - tk.chunk0) * 1024;
     const double* sp = src + (int64_t)v * s_vs + tk.src_off;
@@ -2186,24 +2526,36 @@ int gemm_max_grid(int prec_in, int tile_class) {
   return num_cu() * 2;
 }
 
+// Which operand a batched launch folds over its vectors (see tile_pos): the
+// columns where all vectors share A (T = L x), the rows where they share B
+// (y = T R^T); the forms of an H_eff apply, the only batched launches.
+// At most 4096 vectors: a folded row or column number stays below 2^31.
+static int fold_of(int tr, int nvec, int64_t a_vs, int64_t b_vs) {
+  if (nvec <= 1 || nvec > 4096) return 0;
+  if (tr == 0 && a_vs == 0 && b_vs != 0) return 1;
+  if (tr == 1 && b_vs == 0 && a_vs != 0) return 2;
+  return 0;
+}
+
 template <typename T, typename TOut, int WT>
 static hipError_t runwave(int tr, const GTask* tasks, int ntasks, const GSeg* segs, int tpv, int nvec, const void* A,
                           int64_t a_vs, const void* B, int64_t b_vs, void* C, int64_t c_vs, hipStream_t st) {
   const int total = tpv * nvec;
   if (total <= 0) return hipSuccess;
-  int grid = num_cu() * (WT == 16 ? 8 : 4);  // 32 (16 per wave) or 16 waves per CU
+  int grid = num_cu() * (sizeof(T) == 4 ? (WT == 16 ? 8 : 5) : (WT == 16 ? 6 : 4));  // what the registers allow
   const int need = (total + 3) / 4;
   if (grid > need) grid = need;
   if (grid >= 8) grid &= ~7;
+  const int fold = fold_of(tr, nvec, a_vs, b_vs);
   const T* a = (const T*)A;
   const T* b = (const T*)B;
   TOut* c = (TOut*)C;
-  switch (tr) {
-    case 0: gemm_wave_kernel<T, TOut, false, false, WT><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-    case 1: gemm_wave_kernel<T, TOut, false, true, WT><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-    case 2: gemm_wave_kernel<T, TOut, true, false, WT><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-    default: gemm_wave_kernel<T, TOut, true, true, WT><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-  }
+  if (fold == 1) gemm_wave_kernel<T, TOut, false, false, WT, 1><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, nvec, a, a_vs, b, b_vs, c, c_vs);
+  else if (fold == 2) gemm_wave_kernel<T, TOut, false, true, WT, 2><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, nvec, a, a_vs, b, b_vs, c, c_vs);
+  else if (tr == 0) gemm_wave_kernel<T, TOut, false, false, WT, 0><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, nvec, a, a_vs, b, b_vs, c, c_vs);
+  else if (tr == 1) gemm_wave_kernel<T, TOut, false, true, WT, 0><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, nvec, a, a_vs, b, b_vs, c, c_vs);
+  else if (tr == 2) gemm_wave_kernel<T, TOut, true, false, WT, 0><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, nvec, a, a_vs, b, b_vs, c, c_vs);
+  else gemm_wave_kernel<T, TOut, true, true, WT, 0><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, nvec, a, a_vs, b, b_vs, c, c_vs);
   return hipGetLastError();
 }
 
@@ -2212,21 +2564,26 @@ static hipError_t run16(int tr, const GTask* tasks, int ntasks, const GSeg* segs
                         int64_t a_vs, const void* B, int64_t b_vs, void* C, int64_t c_vs, hipStream_t st) {
   const int total = tpv * nvec;
   if (total <= 0) return hipSuccess;
-  // persistent workgroups per CU: the small tiles (64x64: 92 VGPRs in FP64,
-  // 64 in FP32; 32x32 fewer) run several per CU so that the short-k tiles of
-  // small sectors overlap their load latency; 128x128 keeps two
-  int grid = num_cu() * (BM == 32 ? 8 : (BM == 64 ? (sizeof(T) == 4 ? 8 : 5) : 2));
+  const int fold = fold_of(tr, nvec, a_vs, b_vs);
+  // persistent workgroups per CU: the small tiles run several per CU so that
+  // the short-k tiles of small sectors overlap their load latency; 128x128
+  // keeps two (its registers and two LDS buffers allow no more)
+  int grid = num_cu() * (BM == 32 ? 8 : (BM == 64 ? (sizeof(T) == 4 ? 8 : 4) : 2));
   if (grid > total) grid = total;
   if (grid >= 8) grid &= ~7;
   const T* a = (const T*)A;
   const T* b = (const T*)B;
   TOut* c = (TOut*)C;
-  switch (tr) {
-    case 0: gemm16_kernel<T, TOut, BM, BN, false, false><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-    case 1: gemm16_kernel<T, TOut, BM, BN, false, true><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-    case 2: gemm16_kernel<T, TOut, BM, BN, true, false><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-    default: gemm16_kernel<T, TOut, BM, BN, true, true><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, a, a_vs, b, b_vs, c, c_vs); break;
-  }
+#define MPSA_K16(TA_, TB_, FOLD_)                                                                            \
+  gemm16_kernel<T, TOut, BM, BN, TA_, TB_, FOLD_><<<grid, 256, 0, st>>>(tasks, ntasks, segs, tpv, total, nvec, \
+                                                                        a, a_vs, b, b_vs, c, c_vs)
+  if (fold == 1) MPSA_K16(false, false, 1);
+  else if (fold == 2) MPSA_K16(false, true, 2);
+  else if (tr == 0) MPSA_K16(false, false, 0);
+  else if (tr == 1) MPSA_K16(false, true, 0);
+  else if (tr == 2) MPSA_K16(true, false, 0);
+  else MPSA_K16(true, true, 0);
+#undef MPSA_K16
   return hipGetLastError();
 }
 

@@ -1,0 +1,61 @@
+"""Batched applies (nvec > 1) at every FP64/FP32 tile class: the vectors of a
+batch are folded into one dimension of each grouped product, so tiles straddle
+vector boundaries at odd block sizes.
+
+Bars: FP64 results equal the single-vector apply bit for bit (same k order per
+element) and the numpy execution of the plan's schedule within 1e-13 relative
+(sums of at most a few hundred products of O(1) terms: n eps ~ 5e-14); FP32
+within 2e-6 of the FP64 result (operands and products rounded once at 2^-24,
+sums of the same length)."""
+import numpy as np
+import pytest
+
+import plan_interp
+import problems
+from mpstools_amd import native
+
+pytestmark = pytest.mark.gpu
+
+
+# block dimensions from 1 up: below, at and across one 16-row sub-tile (xxz),
+# thousands of tiny blocks (hubbard), blocks over several tiles (dense, odd)
+@pytest.mark.parametrize("model,L,N,D,seed,dense,nvecs", [
+    ("xxz", 12, 6, 40, 901, False, (2, 17)), ("hubbard", 8, 8, 60, 902, False, (3, 16)),
+    ("tv", 16, 8, 90, 903, False, (5, 64)), ("xxz", 14, 0, 67, 904, True, (2, 3))])
+def test_folded_batches(gpu, oracle, model, L, N, D, seed, dense, nvecs):
+    torch = gpu
+    P = problems.build(oracle, model, L, N, D, seed, dense=dense)
+    c, mpo, itk = P["c"], P["mpo"], P["itk"]
+    Lb, Rb = P["Ls"][c - 1], P["Rs"][c + 2]
+    Lt, Rt, xt = native.Table.from_blocks(Lb), native.Table.from_blocks(Rb), native.Table.from_blocks(P["psi"])
+    vt = xt.union(native.heff2_outkeys(Lt, Rt, xt, mpo[c], mpo[c + 1], itk[c], itk[c + 1]))
+    dL, dR = torch.from_numpy(Lt.pack(Lb)).cuda(), torch.from_numpy(Rt.pack(Rb)).cuda()
+    rng = np.random.default_rng(seed)
+    stride = vt.total + 5  # odd: vectors start at every alignment
+    for prec in (native.F64, native.F32):
+        plan = native.HeffPlan(Lt, Rt, vt, vt, (mpo[c], mpo[c + 1]), (itk[c], itk[c + 1]), prec)
+        plan.bind_env(dL, dR)
+        for nvec in nvecs:
+            x = rng.standard_normal((nvec, stride))
+            ref = np.zeros((nvec, vt.total))
+            ref_plan = native.HeffPlan(Lt, Rt, vt, vt, (mpo[c], mpo[c + 1]), (itk[c], itk[c + 1]), native.F64)
+            for v in range(nvec):
+                plan_interp.run_heff(ref_plan.describe(), Lt.pack(Lb), Rt.pack(Rb), x[v, :vt.total], ref[v],
+                                     ref_plan.info()["workspace_bytes"] // 8)
+            dx = torch.from_numpy(x).cuda()
+            for cls in range(5):
+                print("[case]", model, prec, nvec, cls, flush=True)
+                plan.set_tile_class(1, cls)
+                plan.set_tile_class(2, cls)
+                dy = torch.full((nvec, stride), 7.0, dtype=torch.float64, device="cuda")
+                plan.apply(dx, dy, nvec, stride, stride)
+                one = torch.full((nvec, stride), 7.0, dtype=torch.float64, device="cuda")
+                for v in range(nvec):
+                    plan.apply(dx[v], one[v])
+                torch.cuda.synchronize()
+                assert torch.equal(dy, one)  # also: nothing written between the vectors
+                blocks = vt.unpack(dy[nvec - 1, :vt.total].cpu().numpy())
+                want = vt.unpack(ref[nvec - 1])
+                num = sum(float(np.sum((blocks[k] - want[k]) ** 2)) for k in want.keys())
+                den = sum(float(np.sum(want[k] ** 2)) for k in want.keys())
+                assert (num / den) ** 0.5 <= (1e-13 if prec == native.F64 else 2e-6), (prec, nvec, cls)
