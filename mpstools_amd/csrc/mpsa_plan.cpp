@@ -252,8 +252,6 @@ static int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 // with zeros to a multiple of 32: the streaming kernel moves whole 32-wide slabs.
 static int64_t pad8(int64_t x) { return (x + 31) & ~int64_t(31); }
 
-// Tile class: the largest workgroup tile that wastes at most 20% of its
-// MFMA work on padding; the smallest tile otherwise.
 // The 256x256 class needs unit scales and per-lane operand offsets
 // (row * ld * 2 bytes inside one block) below 2^31.
 static bool fits_pipe_tile(const std::vector<GTask>& t, const std::vector<GSeg>& segs) {
@@ -267,49 +265,68 @@ static bool fits_pipe_tile(const std::vector<GTask>& t, const std::vector<GSeg>&
   return true;
 }
 
+// The wave tiles (FP64/FP32 classes 3 and 4) index k-steps times a leading
+// dimension with 24-bit factors.
+static bool fits_wave_tile(const std::vector<GSeg>& segs) {
+  for (auto& g : segs)
+    if (g.lda >= (1 << 24) || g.ldb >= (1 << 24)) return false;
+  return true;
+}
+
 // Tile classes a stage may launch with: every class of the precision, the
-// 256x256 class only where fits_pipe_tile holds.
+// 256x256 class only where fits_pipe_tile holds, the wave tiles only where
+// fits_wave_tile does.
 static bool class_admissible(const std::vector<GTask>& t, const std::vector<GSeg>& segs, int prec, int cls) {
   if (cls < 0 || cls >= num_tile_classes(prec)) return false;
   const bool bf = prec == BF16 || prec == BF16X3;
-  return !bf || cls != 3 || fits_pipe_tile(t, segs);
+  if (bf) return cls != 3 || fits_pipe_tile(t, segs);
+  return cls < 3 || fits_wave_tile(segs);
 }
 
+// The tile class of a stage without tuning, from its blocks' shapes.  A large
+// tile reads fewer operand bytes per MFMA; it is taken where it is mostly
+// full and the launch has tiles enough for 256 CUs.  Measured on one MI355X
+// (us per stage, dense bonds of dimension D unless named; tiles in brackets):
+//   FP64 128x128 / 64x64: D = 2048 stage 2 4180 [1024] / 4760, D = 1500 stage 1
+//     1970 [1440] / 2010, stage 2 3110 [576: 2.25 rounds of 256] / 2570,
+//     D = 1024 stage 2 678 [256] / 589: 128x128 from 512 tiles whose rounds
+//     of 256 are at least 80 % full;
+//   FP64 64x64 / 32x32: D = 400 stage 1 72 [490] / 92, stage 2 195 [196] / 127,
+//     D = 777 510 [676] / 583, D = 100 30 [16] / 15: 64x64 from 400 tiles;
+//   BF16X3 256x256 / 64x64: D = 2048 560 / 1610, D = 1024 stage 1 82 [160] /
+//     235, stage 2 199 [64] / 184, D = 500 stage 1 47 [40] / 29, stage 2 110
+//     [16] / 49: 256x256 from 128 tiles, the other large tiles from 512;
+//   BF16X3 64x64 / 32x32: t-V sectors of 20-120 rows, 64 vectors 430 / 846,
+//     of 1-80 rows 105 / 137, Hubbard sectors of 1-31 rows, 16 vectors 319 /
+//     254: 32x32 only where 64x64 is less than 12 % full;
+//   FP64 32x32 / 16x16 wave tile: Hubbard, 16 vectors 937 / 524, XXZ sectors of
+//     1-196 rows 43 / 50: the wave tile where 32x32 is less than 40 % full.
 static int pick_class(const std::vector<GTask>& t, const std::vector<GSeg>& segs, int prec) {
-  int best = -1, fallback = 1;
-  int best_area = 0;
-  double fallback_fill = -1.0;
-  const bool pipe_ok = fits_pipe_tile(t, segs);
   const bool bfp = prec == BF16 || prec == BF16X3;
-  double fill_cls[kMaxTileClasses] = {0, 0, 0, 0, 0};
+  double fill[kMaxTileClasses] = {0, 0, 0, 0, 0};
+  double tiles[kMaxTileClasses] = {0, 0, 0, 0, 0};
   for (int cls = 0; cls < num_tile_classes(prec); ++cls) {
-    if (bfp && cls == 3 && !pipe_ok) continue;
     int bm, bn;
     tile_dims(prec, cls, &bm, &bn);
     double useful = 0, padded = 0;
     for (auto& x : t) {
+      const double nt = (double)((x.m + bm - 1) / bm) * ((x.n + bn - 1) / bn);
       useful += (double)x.m * x.n;
-      padded += (double)((x.m + bm - 1) / bm) * ((x.n + bn - 1) / bn) * (double)bm * bn;
+      padded += nt * bm * bn;
+      tiles[cls] += nt;
     }
-    const double fill = padded > 0 ? useful / padded : 1.0;
-    fill_cls[cls] = fill;
-    if (!bfp && cls >= 3) continue;  // the wave tiles: decided below (class 4 by the autotuner only)
-    if (fill >= 0.8 && bm * bn > best_area) {
-      best = cls;
-      best_area = bm * bn;
-    }
-    if (fill > fallback_fill) {  // no tile fills 80 %: the least padded one
-      fallback = cls;
-      fallback_fill = fill;
-    }
+    fill[cls] = padded > 0 ? useful / padded : 1.0;
   }
-  const int pick = best >= 0 ? best : fallback;
-  // FP64/FP32 stages of blocks mostly below 16 rows or columns (the 32x32
-  // tile under 40 % full): the barrier-free 16x16 wave tile (measured 1.9x
-  // on the 16-vector Hubbard D = 1024 bond, slower than 32x32 on the t-V and
-  // XXZ bonds whose blocks reach 80 and 196)
-  if (!bfp && pick == 2 && fill_cls[2] < 0.4) return 3;
-  return pick;
+  if (bfp) {
+    if (fill[3] >= 0.8 && tiles[3] >= 128 && fits_pipe_tile(t, segs)) return 3;
+    if (fill[0] >= 0.8 && tiles[0] >= 512) return 0;
+    if (fill[2] >= 0.8 && tiles[2] >= 512) return 2;
+    return fill[1] < 0.12 ? 4 : 1;
+  }
+  const double rounds = std::ceil(tiles[0] / 256.0);
+  if (fill[0] >= 0.8 && tiles[0] >= 512 && tiles[0] >= 0.8 * 256.0 * rounds) return 0;
+  if (fill[1] >= 0.75 && tiles[1] >= 400) return 1;
+  return fill[2] < 0.4 && fits_wave_tile(segs) ? 3 : 2;
 }
 
 // Number the workgroup tiles of a stage for tile class cls, in task order
