@@ -46,6 +46,7 @@
 #include "../../include/mpstools_amd.h"
 #include "mpsa_host.h"
 #include "mpsa_internal.h"
+#include "mpsa_svd.h"
 
 using namespace mpsa;
 using namespace mpsa::host;
@@ -660,69 +661,25 @@ void big_factor(Eng& E, bool qr, bool left, int64_t m, int64_t n, double* M, int
   hchk(launch_fill(Sv, k, 1.0, E.st), "cheb: unit S");
 }
 
-// Chunk table of launch_house_panels / launch_house_apply: sector s has its
-// workgroups at base[s] .. base[s + 1]; returns the largest min(m, n).
-int house_table(const std::vector<SvdTask>& ts, int layout, std::vector<int>& base) {
-  base.assign(ts.size() + 1, 0);
-  int kmax = 0;
-  for (size_t i = 0; i < ts.size(); ++i) {
-    base[i + 1] = base[i] + house_chunks(ts[i].m, ts[i].n, layout);
-    kmax = std::max(kmax, (int)std::min(ts[i].m, ts[i].n));
+// svd_blocked_run's device services over the engine's pool and stream.
+struct SvdDev {
+  Eng& E;
+  std::vector<Buf> held;
+  template <typename T>
+  const void* put(const std::vector<T>& v) {
+    held.push_back(E.upload(v));
+    return held.back().p;
   }
-  return kmax;
-}
+  void check(hipError_t e, const char* what) { hchk(e, what); }
+  void wait() { E.sync(); }
+};
 
-// The SVD of the large sectors in phases (mpsa_factor.hip): the load, the
-// reflections in panels over several workgroups per sector, the init, sweeps
-// of block-tournament rounds until a sweep rotates nothing (one host wait per
-// sweep), the back-transform over several workgroups, the outputs.
+// The SVD of the large sectors (svd_blocked_run).
 void svd_blocked(Eng& E, bool cplx, const std::vector<SvdTask>& big, const double* M, int64_t m_plane, double* U,
                  int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W, int64_t w_plane) {
-  const int nb = (int)big.size();
-  std::vector<int> hbase;
-  const int kmax = house_table(big, 0, hbase);
-  Buf dt = E.upload(big), dh = E.upload(hbase);
-  Buf flags(E.pool, nb, E.st);
-  const SvdTask* t = (const SvdTask*)dt.p;
-  auto phase = [&](int ph, const char* what) {
-    hchk(launch_svd_phase(cplx, ph, t, nb, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane, E.st), what);
-  };
-  phase(kPhLoad, "cheb: sector SVD load");
-  hchk(launch_house_panels(cplx, 0, t, nb, (const int*)dh.p, hbase.back(), kmax, W, w_plane, E.st),
-       "cheb: sector SVD reflections");
-  phase(kPhInit, "cheb: sector SVD init");
-  // sweeps over the sectors still rotating: a sweep that rotates nothing in a
-  // sector leaves it as it is, so later sweeps would not rotate it either
-  std::vector<SvdTask> act = big;
-  std::vector<double> hf((size_t)nb);
-  for (int sweep = 0; sweep < 60 && !act.empty(); ++sweep) {
-    const int na = (int)act.size();
-    std::vector<int> base((size_t)na + 1, 0);
-    int rounds = 0, rmax = 1;
-    for (int i = 0; i < na; ++i) {
-      const SvdTask& a = act[(size_t)i];
-      base[(size_t)i + 1] = base[(size_t)i] + svd_block_pairs(a.m, a.n);
-      rounds = std::max(rounds, svd_block_rounds(a.m, a.n));
-      rmax = std::max(rmax, (int)std::min(a.m, a.n));
-    }
-    Buf da = E.upload(act), db = E.upload(base);
-    for (int round = -1; round < rounds; ++round)
-      hchk(launch_svd_block_round(cplx, (const SvdTask*)da.p, na, (const int*)db.p, base.back(), round, W, w_plane,
-                                  flags.p, rmax, E.st),
-           "cheb: sector SVD round");
-    hchk(hipMemcpyAsync(hf.data(), flags.p, sizeof(double) * (size_t)na, hipMemcpyDeviceToHost, E.st),
-         "cheb: sector SVD flags");
-    E.sync();
-    std::vector<SvdTask> next;
-    for (int i = 0; i < na; ++i)
-      if (hf[(size_t)i] != 0.0) next.push_back(act[(size_t)i]);
-    act.swap(next);
-    if (!act.empty()) hchk(launch_fill(flags.p, na, 0.0, E.st), "cheb: sector SVD flags");
-  }
-  phase(kPhBackInit, "cheb: sector SVD back-transform");
-  hchk(launch_house_apply(cplx, 0, t, nb, (const int*)dh.p, hbase.back(), W, w_plane, E.st),
-       "cheb: sector SVD back-transform");
-  phase(kPhOut, "cheb: sector SVD outputs");
+  Buf flags(E.pool, (int64_t)big.size(), E.st);
+  SvdDev dev{E, {}};
+  svd_blocked_run(dev, cplx, big, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane, flags.p, E.st);
 }
 
 // The QR (right = 0) or LQ (right = 1) of the large sectors the same way:

@@ -8,9 +8,10 @@
 //
 // Per centre charge qc = l + q(s1) the blocks (l, r, (s1, s2)) are gathered
 // into one dense matrix (rows by s1 ascending, columns by s2 ascending), its
-// SVD is taken in FP64 by Jacobi (rocSOLVER gesvdj: the factorisation of the
-// reference's dgesvd, backward stable), the sign of every singular pair is
-// fixed by FixPhase, and the global truncation runs on the host over all
+// SVD is taken in FP64 by one-sided Jacobi (this library's batched kernels, all
+// sectors at once; rocSOLVER's gesvdj for sectors beyond their limits; both
+// backward stable, as the reference's dgesvd), the sign of every singular pair
+// is fixed by FixPhase, and the global truncation runs on the host over all
 // sectors' singular values exactly as the reference orders them.
 // Sectors with min(m, n) >= kPrecondMin (the dense D = 2048 bond's 4096 x 4096
 // sector) of a count-limited split (chimax below the number of singular
@@ -55,6 +56,7 @@
 
 #include "../../include/mpstools_amd.h"
 #include "mpsa_internal.h"
+#include "mpsa_svd.h"
 
 using namespace mpsa;
 
@@ -86,6 +88,18 @@ constexpr int64_t kPrecondMin = MPSA_PRECOND_MIN;
 constexpr double kDmZero = 1e-10;
 constexpr double kDmTail = 1e-4;
 
+// Sectors of at most kOwnMaxR singular values and kOwnMaxP rows or columns (at
+// most kVecRowsMax from kOwnBlockR singular values on, where several
+// workgroups share a sector) go to the library's batched one-sided Jacobi SVD
+// (mpsa_factor.hip), all of them in the same launches; larger ones to
+// rocSOLVER's gesvdj, one call and one wait each.  The t-V D = 512 bond (16
+// sectors of up to 160 x 160): 166 ms by gesvdj, 7.6 ms here.
+constexpr int64_t kOwnBlockR = 32, kOwnMaxR = kSvdBlockMaxR, kOwnMaxP = 4096;
+bool own_svd(int64_t m, int64_t n) {
+  const int64_t r = std::min(m, n), p = std::max(m, n);
+  return r <= kOwnMaxR && p <= (r < kOwnBlockR ? kOwnMaxP : (int64_t)kVecRowsMax);
+}
+
 // one rocBLAS handle per device, created on first use
 rocblas_handle handle_for_current_device() {
   static std::map<int, rocblas_handle> handles;
@@ -111,6 +125,33 @@ struct DevArr {
   ~DevArr() {
     if (p) (void)hipFree(p);
   }
+};
+
+// svd_blocked_run's device services: chunks of device memory and the host
+// sources of the copies into them, both kept until the end of the call.
+struct SvdDev {
+  static constexpr size_t kChunk = 1 << 18;
+  hipStream_t st;
+  std::vector<std::unique_ptr<DevArr<char>>> chunks;
+  std::vector<std::vector<char>> src;
+  size_t at = 0, cap = 0;
+  template <typename T>
+  const void* put(const std::vector<T>& v) {
+    const size_t bytes = sizeof(T) * v.size();
+    if (at + bytes > cap) {
+      cap = std::max(kChunk, bytes);
+      chunks.emplace_back(new DevArr<char>());
+      chunks.back()->alloc(cap);
+      at = 0;
+    }
+    char* p = chunks.back()->p + at;
+    at = (at + bytes + 255) / 256 * 256;
+    src.emplace_back((const char*)v.data(), (const char*)v.data() + bytes);
+    if (bytes) hchk(hipMemcpyAsync(p, src.back().data(), bytes, hipMemcpyHostToDevice, st), "split: upload");
+    return p;
+  }
+  void check(hipError_t e, const char* what) { hchk(e, what); }
+  void wait() { hchk(hipStreamSynchronize(st), "split: sync"); }
 };
 
 struct Sector {
@@ -230,8 +271,12 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
       hchk(launch_copy2d(dg.p, (int)gather.size(), maxel, dpsi, M.p, nullptr, st), "split: gather");
     }
     // SVD + FixPhase per sector (BoostSVD, lapack_routines.cpp:614-634)
-    rocblas_handle h = handle_for_current_device();
-    rchk(rocblas_set_stream(h, st), "rocblas_set_stream");
+    rocblas_handle h = nullptr;  // made when a sector needs it
+    auto need_handle = [&]() {
+      if (h) return;
+      h = handle_for_current_device();
+      rchk(rocblas_set_stream(h, st), "rocblas_set_stream");
+    };
     // Sectors with min(m, n) >= kPrecondMin take the density-matrix route:
     // the Gram matrix of the side that stays a bare isometry (rho = M M^T
     // when lambda goes right, G = M^T M when it goes left) is diagonalised by
@@ -282,13 +327,51 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
       hchk(hipStreamSynchronize(st), "split: sync");
       if (ih != 0) throw SErr(MPSA_EINVAL, std::string("split: ") + what + " did not converge (info " + std::to_string(ih) + ")");
     };
+    // the sectors of the batched Jacobi SVD, largest first
+    std::vector<SvdTask> small, blocked;
+    int64_t w_total = 0;
+    for (auto& kv : secs) {
+      const Sector& S = kv.second;
+      if (S.k == 0 || dm_route(S) || !own_svd(S.m, S.n)) continue;
+      SvdTask t{};
+      t.a_off = S.off_M;
+      t.u_off = S.off_U;
+      t.vt_off = S.off_V;
+      t.s_off = S.off_S;
+      t.w_off = w_total;
+      t.m = (int32_t)S.m;
+      t.n = (int32_t)S.n;
+      t.lda = (int32_t)S.m;
+      w_total += align64(svd_workspace(S.m, S.n));
+      (S.k >= kOwnBlockR ? blocked : small).push_back(t);
+    }
+    SvdDev dev{st, {}, {}, 0, 0};
+    DevArr<double> Wk, flags;
+    if (w_total) {
+      const auto larger = [](const SvdTask& a, const SvdTask& b) {
+        return (int64_t)a.m * a.n * std::min(a.m, a.n) > (int64_t)b.m * b.n * std::min(b.m, b.n);
+      };
+      std::stable_sort(small.begin(), small.end(), larger);
+      std::stable_sort(blocked.begin(), blocked.end(), larger);
+      Wk.alloc((size_t)w_total);
+      if (!small.empty())
+        hchk(launch_svd_batched(0, (const SvdTask*)dev.put(small), (int)small.size(), M.p, 0, U.p, 0, V.p, 0, Sg.p,
+                                Wk.p, 0, st),
+             "split: sector SVD");
+      if (!blocked.empty()) {
+        flags.alloc(blocked.size());
+        hchk(launch_fill(flags.p, (int64_t)blocked.size(), 0.0, st), "split: flags");
+        svd_blocked_run(dev, false, blocked, M.p, 0, U.p, 0, V.p, 0, Sg.p, Wk.p, 0, flags.p, st);
+      }
+    }
     const double one = 1.0, zero = 0.0;
     std::vector<std::vector<double>> big_sig;    // host sources of the sorted sigmas, alive until the final sync
     std::vector<std::vector<Copy2D>> big_moves;  // host sources of the gather tasks, likewise
     std::vector<std::unique_ptr<DevArr<Copy2D>>> big_dmoves;
     for (auto& kv : secs) {
       Sector& S = kv.second;
-      if (S.k == 0) continue;
+      if (S.k == 0 || (!dm_route(S) && own_svd(S.m, S.n))) continue;
+      need_handle();
       const rocblas_int m = (rocblas_int)S.m, n = (rocblas_int)S.n, k = (rocblas_int)S.k;
       double* Ms = M.p + S.off_M;
       if (dm_route(S)) {

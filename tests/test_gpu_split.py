@@ -217,3 +217,38 @@ def test_split_density_route_count_limited(gpu, oracle, direction, chimax, kept)
     got, want = twosite(gl, gr), twosite(left, right)
     assert got.keys() == want.keys()
     assert max(np.max(np.abs(got[k] - want[k])) for k in want.keys()) <= 1e-9
+
+
+@pytest.mark.parametrize("dl,dr", [(1, 1), (1, 20), (15, 16), (16, 16), (17, 33), (40, 16), (16, 512), (16, 513),
+                                   (4, 2048), (4, 2049), (256, 256), (257, 256)])
+@pytest.mark.parametrize("direction", [1, 0])
+def test_split_at_the_limits_of_the_batched_svd(gpu, dl, dr, direction):
+    """One dense 2 dl x 2 dr sector on either side of the lines of the sector
+    SVD's dispatch (one workgroup below 32 singular values, several from 32 to
+    512 with at most 1024 rows, rocSOLVER beyond), against numpy's SVD.  Full
+    rank with singular values 1 .. 2^-k, k < 8, so every vector is determined:
+    bars as in _cmp_lambda, the rebuilt state and the isometry within 1e-12
+    (n eps is below 1e-12 up to n = 4096)."""
+    torch = gpu
+    _say("split limits", 2 * dl, "x", 2 * dr, "direction", direction)
+    from mpstools_amd.blocks import Blocks
+    rng = np.random.default_rng(1000 * dl + dr)
+    m, n = 2 * dl, 2 * dr
+    k = min(m, n)
+    U = np.linalg.qr(rng.standard_normal((m, k)))[0]
+    V = np.linalg.qr(rng.standard_normal((n, k)))[0]
+    M = (U * 2.0 ** (-8.0 * np.arange(k) / k)) @ V.T
+    M /= np.linalg.norm(M)
+    psi = Blocks(2)
+    for s1 in range(2):
+        for s2 in range(2):
+            psi[(0, 0, s1, s2)] = M[s1 * dl:(s1 + 1) * dl, s2 * dr:(s2 + 1) * dr]
+    t = native.Table.from_blocks(psi)
+    out = native.split(t, torch.from_numpy(t.pack(psi)).cuda(), [0, 0], [0, 0], direction=direction, chimax=10 ** 6)
+    assert out["chi"] == k
+    _cmp_lambda(out["lam"], {0: np.linalg.svd(M, compute_uv=False)})
+    _check_isometry(out["left" if direction > 0 else "right"], out["lam"], "left" if direction > 0 else "right", 1e-12)
+    gl = out["left"][0].unpack(out["left"][1].cpu().numpy())
+    gr = out["right"][0].unpack(out["right"][1].cpu().numpy())
+    got = twosite(gl, gr)
+    assert max(np.max(np.abs(got[key] - psi[key])) for key in psi.keys()) <= 1e-12
