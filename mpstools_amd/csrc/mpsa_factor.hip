@@ -41,10 +41,26 @@ namespace {
 constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
 
+// Sum over the 64 lanes of a wave (all active), in every lane: moves inside
+// the vector unit (rows of 16 lanes, then across rows) instead of six trips
+// through the LDS crossbar, which a Jacobi rotation or reflection waits for
+// one after another.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROWS, 0xf, false);
+  return x + __hiloint2double(hi, lo);
+}
 __device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
+  x = dpp_add<0x111, 0xf>(x);  // row_shr 1, 2, 4, 8: lane 15 of a row holds its sum
+  x = dpp_add<0x112, 0xf>(x);
+  x = dpp_add<0x114, 0xf>(x);
+  x = dpp_add<0x118, 0xf>(x);
+  x = dpp_add<0x142, 0xa>(x);  // row_bcast 15: rows 0 and 2 into rows 1 and 3
+  x = dpp_add<0x143, 0xc>(x);  // row_bcast 31: row 1 into rows 2 and 3
+  const int lo = __builtin_amdgcn_readlane(__double2loint(x), 63);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(x), 63);
+  return __hiloint2double(hi, lo);
 }
 
 // Column j of a p-row matrix with leading dimension ld, planar complex.
