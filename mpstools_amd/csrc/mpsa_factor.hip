@@ -97,6 +97,48 @@ __device__ __forceinline__ void rotate_cols(const Mat<C>& X, int p, int i, int j
   }
 }
 
+// The Jacobi rotation (c, sn, phase er + i ei) that makes columns of squared
+// norms a and b and inner product gr + i gi orthogonal, in every lane; false
+// when |g| <= tol sqrt(a b) (nothing to rotate).  t = h / (|d| + sqrt(d^2 + h^2))
+// with d = b - a, h = 2 |g| is the smaller root of the rotation's quadratic; two
+// square roots and one division, where the quotient form takes three of each
+// in a chain that a whole round waits for.  Columns whose products could leave
+// the range of doubles take that form.
+template <bool C>
+__device__ __forceinline__ bool jacobi_rotation(double a, double b, double gr, double gi, double tol, double& c,
+                                                double& sn, double& er, double& ei) {
+  if (a == 0.0 || b == 0.0) return false;
+  if (a > 1e-120 && b > 1e-120 && a < 1e120 && b < 1e120) {
+    const double g2 = gr * gr + (C ? gi * gi : 0.0);
+    if (!(g2 > tol * tol * (a * b))) return false;
+    double g;
+    if (C) {
+      const double ig = rsqrt(g2);
+      er = gr * ig;
+      ei = gi * ig;
+      g = g2 * ig;
+    } else {
+      er = gr < 0.0 ? -1.0 : 1.0;
+      ei = 0.0;
+      g = fabs(gr);
+    }
+    const double d = b - a, h = 2.0 * g;
+    const double t = (d >= 0.0 ? h : -h) / (fabs(d) + sqrt(d * d + h * h));
+    c = rsqrt(1.0 + t * t);
+    sn = c * t;
+    return true;
+  }
+  const double g = C ? hypot(gr, gi) : fabs(gr);
+  if (!(g > tol * (sqrt(a) * sqrt(b)))) return false;
+  er = gr / g;
+  ei = C ? gi / g : 0.0;
+  const double zeta = (b - a) / (2.0 * g);
+  const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
+  c = 1.0 / sqrt(1.0 + t * t);
+  sn = c * t;
+  return true;
+}
+
 // Rows per lane of the register-held column paths: a column of up to
 // 64 * kRpl rows lives in registers of one wave while it is reduced and
 // updated (one global read and one write instead of two reads and a write),
@@ -460,12 +502,8 @@ __device__ __forceinline__ void jacobi_small(double* ar, double* ai, double* wr,
         const double a = wave_sum(xir * xir + xii * xii), b = wave_sum(xjr * xjr + xji * xji);
         const double gr = wave_sum(xir * xjr + xii * xji);
         const double gi = C ? wave_sum(xir * xji - xii * xjr) : 0.0;  // a_i^H a_j
-        const double g = C ? sqrt(gr * gr + gi * gi) : fabs(gr);
-        if (!(g > tol * sqrt(a * b)) || a == 0.0 || b == 0.0) continue;
-        const double er = gr / g, ei = C ? gi / g : 0.0;
-        const double zeta = (b - a) / (2.0 * g);
-        const double tt = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-        const double c = 1.0 / sqrt(1.0 + tt * tt), sn = c * tt;
+        double c, sn, er, ei;
+        if (!jacobi_rotation<C>(a, b, gr, gi, tol, c, sn, er, ei)) continue;
         // x_i' = c x_i - s conj(e) x_j, x_j' = s e x_i + c x_j (as rotate_cols)
         if (lane < r) {
           const double yir = wr[i * r + lane], yjr = wr[j * r + lane];
@@ -496,6 +534,7 @@ __device__ __forceinline__ void jacobi_small(double* ar, double* ai, double* wr,
   }
 }
 
+static_assert(kSmallRows == 512 && kSmallCols == 64 && kQrLds + 6 * kSmallCols <= 8192, "qr_in_lds states these limits");
 // LDS doubles of X: p r elements (both planes) of at most cap
 __device__ __forceinline__ bool small_fits(int p, int r, bool cplx, int64_t cap) {
   return p <= kSmallRows && r <= kSmallCols && (int64_t)p * r * (cplx ? 2 : 1) <= cap;
@@ -657,12 +696,8 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
         b = wave_sum(b);
         gr = wave_sum(gr);
         if (C) gi = wave_sum(gi);
-        const double g = C ? sqrt(gr * gr + gi * gi) : fabs(gr);
-        if (!(g > tol * sqrt(a * b)) || a == 0.0 || b == 0.0) continue;
-        const double er = gr / g, ei = C ? gi / g : 0.0;
-        const double zeta = (b - a) / (2.0 * g);
-        const double tt = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-        const double c = 1.0 / sqrt(1.0 + tt * tt), s = c * tt;
+        double c, s, er, ei;
+        if (!jacobi_rotation<C>(a, b, gr, gi, tol, c, s, er, ei)) continue;
         // a_i' = c a_i - s conj(e) a_j, a_j' = s e a_i + c a_j (as rotate_cols)
 #pragma unroll
         for (int q = 0; q < kRpl; ++q) {
@@ -870,12 +905,12 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
 // After the reduction and init phases the r columns of A = R^H are
 // split into blocks of kBj columns; one launch runs one round of the block
 // tournament over every large sector at once, one workgroup per block pair
-// (I, J): it loads the 2 kBj columns into LDS, rotates every pair (i in I,
-// j in J) once with the scalar kernel's rotation and threshold, writes them
+// (I, J) (svd_block_across_kernel): it rotates every pair (i in I, j in J)
+// once with the scalar kernel's rotation and threshold, writes the columns
 // back and applies the accumulated 2 kBj x 2 kBj rotation to the same columns
-// of Wm.  The launch with round < 0 does the pairs inside each block (a
-// tournament over its columns, one workgroup per block), so a sweep (that
-// launch, then the rounds) visits every pair of columns once.  Sectors have
+// of Wm.  The launch with round < 0 (svd_block_inner_kernel) does the pairs
+// inside each block (a tournament over its columns, one workgroup per block),
+// so a sweep (that launch, then the rounds) visits every pair of columns once.  Sectors have
 // their block pairs at pair_base[s] .. pair_base[s + 1] of the grid (twice
 // that for the intra-block launch); rotated[s] is set when any pair of the
 // sector rotated (the host repeats sweeps until none does, then the
@@ -885,22 +920,21 @@ constexpr int kBjMaxR = 512;
 static_assert(kBj == kWaves, "one wave per column of block I in the rounds across blocks");
 
 template <bool C>
-__global__ __launch_bounds__(kThreads) void svd_block_round_kernel(const SvdTask* __restrict__ tasks, int ntasks,
-                                                                   const int* __restrict__ pair_base, int round,
+__global__ __launch_bounds__(kThreads) void svd_block_inner_kernel(const SvdTask* __restrict__ tasks, int ntasks,
+                                                                   const int* __restrict__ pair_base,
                                                                    double* __restrict__ W, int64_t w_plane,
                                                                    double* __restrict__ rotated, int rmax) {
-  // the block pair's columns: 2 kBj x rmax per plane of dynamic LDS (rmax: the
-  // launch's largest r, so that small launches fit two workgroups per CU)
+  // the block's columns: kBj x rmax per plane of dynamic LDS (rmax: the
+  // launch's largest r, so that small launches fit several workgroups per CU)
   extern __shared__ double blk_lds[];
   double* const Lr = blk_lds;
-  double* const Li = blk_lds + 2 * kBj * rmax;
-  __shared__ double Vr[2 * kBj * 2 * kBj], Vi[2 * kBj * 2 * kBj];
+  double* const Li = blk_lds + kBj * rmax;
+  __shared__ double Vr[kBj * kBj], Vi[kBj * kBj];
   __shared__ int any;
-  // sector of this workgroup: pair_base is ascending, pair_base[0] = 0; the
-  // intra-block launch (round < 0) has two workgroups per block pair slot
+  // sector of this workgroup: pair_base is ascending, pair_base[0] = 0; two
+  // workgroups per block pair slot
   int lo = 0, hi = ntasks - 1;
-  const bool intra = round < 0;
-  const int b = blockIdx.x, bs = intra ? b >> 1 : b;
+  const int b = blockIdx.x, bs = b >> 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (pair_base[mid] <= bs) lo = mid;
@@ -908,34 +942,18 @@ __global__ __launch_bounds__(kThreads) void svd_block_round_kernel(const SvdTask
   }
   const int sidx = lo;
   const SvdTask t = tasks[sidx];
-  const int q = b - (intra ? 2 : 1) * pair_base[sidx];
+  const int q = b - 2 * pair_base[sidx];
   const int m = t.m, n = t.n;
   const int p = m < n ? n : m, r = m < n ? m : n;
-  const int nb = (r + kBj - 1) / kBj, nbb = nb + (nb & 1);
-  if (r > rmax) return;
-  int I, J;
-  if (intra) {  // the pairs inside block q
-    if (q >= nb) return;
-    I = q;
-    J = nb;
-  } else {  // the pairs across blocks I and J of the tournament's round
-    if (round >= nbb - 1 || q >= nbb / 2) return;
-    I = (round + q) % (nbb - 1);
-    J = q == 0 ? nbb - 1 : (round + nbb - 1 - q) % (nbb - 1);
-    if (I > J) {
-      const int x = I;
-      I = J;
-      J = x;
-    }
-    if (J >= nb) return;  // the bye of an odd block count
-  }
+  const int nb = (r + kBj - 1) / kBj;
+  if (r > rmax || q >= nb) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int i0 = I * kBj, wI = min(kBj, r - i0), j0 = J * kBj, wJ = J < nb ? min(kBj, r - j0) : 0, w = wI + wJ;
-  auto colof = [&](int c) { return c < wI ? i0 + c : j0 + (c - wI); };
+  const int i0 = q * kBj, w = min(kBj, r - i0);
+  auto colof = [&](int c) { return i0 + c; };
   const int64_t o_wm = (int64_t)p * r, o_a = 2 * (int64_t)p * r + (int64_t)r * r;
   Mat<C> Wm{W + t.w_off + o_wm, W + t.w_off + o_wm + w_plane, r};
   Mat<C> A{W + t.w_off + o_a, W + t.w_off + o_a + w_plane, r};
-  // the block pair's columns of A into LDS (column c at c * r), V = identity
+  // the block's columns of A into LDS (column c at c * r), V = identity
   for (int e = tid; e < w * r; e += kThreads) {
     const int c = e / r, row = e - c * r;
     Lr[c * r + row] = A.r(row, colof(c));
@@ -949,24 +967,15 @@ __global__ __launch_bounds__(kThreads) void svd_block_round_kernel(const SvdTask
   __syncthreads();
   const double tol = sqrt((double)r) * DBL_EPSILON;
   const int ww = w + (w & 1);
-  // intra: a tournament over the block's wI columns; across: kBj sub-rounds,
-  // wave a pairs column a of I with column (a + sub) mod kBj of J
-  const int nsub = intra ? ww - 1 : kBj;
-  for (int sub = 0; sub < nsub; ++sub) {
-    for (int pq = wave; pq < (intra ? ww / 2 : kBj); pq += kWaves) {
-      int i, j;
-      if (intra) {
-        i = (sub + pq) % (ww - 1);
-        j = pq == 0 ? ww - 1 : (sub + ww - 1 - pq) % (ww - 1);
-        if (i > j) {
-          const int x = i;
-          i = j;
-          j = x;
-        }
-      } else {
-        i = pq;
-        j = wI + (pq + sub) % kBj;
-        if (i >= wI) continue;
+  // a tournament over the block's columns
+  for (int sub = 0; sub < ww - 1; ++sub) {
+    for (int pq = wave; pq < ww / 2; pq += kWaves) {
+      int i = (sub + pq) % (ww - 1);
+      int j = pq == 0 ? ww - 1 : (sub + ww - 1 - pq) % (ww - 1);
+      if (i > j) {
+        const int x = i;
+        i = j;
+        j = x;
       }
       if (j >= w) continue;
       double a = 0.0, bb = 0.0, gr = 0.0, gi = 0.0;
@@ -987,12 +996,8 @@ __global__ __launch_bounds__(kThreads) void svd_block_round_kernel(const SvdTask
       bb = wave_sum(bb);
       gr = wave_sum(gr);
       if (C) gi = wave_sum(gi);
-      const double g = C ? sqrt(gr * gr + gi * gi) : fabs(gr);
-      if (!(g > tol * sqrt(a * bb)) || a == 0.0 || bb == 0.0) continue;
-      const double er = gr / g, ei = C ? gi / g : 0.0;
-      const double zeta = (bb - a) / (2.0 * g);
-      const double tt = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-      const double c = 1.0 / sqrt(1.0 + tt * tt), sn = c * tt;
+      double c, sn, er, ei;
+      if (!jacobi_rotation<C>(a, bb, gr, gi, tol, c, sn, er, ei)) continue;
       // a_i' = c a_i - s conj(e) a_j, a_j' = s e a_i + c a_j (as rotate_cols), on the columns and on V
       for (int row = lane; row < r; row += 64) {
         const double xir = Lr[i * r + row], xjr = Lr[j * r + row];
@@ -1037,16 +1042,16 @@ __global__ __launch_bounds__(kThreads) void svd_block_round_kernel(const SvdTask
     if (C) A.m(row, colof(c)) = Li[c * r + row];
   }
   for (int row = tid; row < r; row += kThreads) {
-    double orr[2 * kBj], oi[2 * kBj];
+    double orr[kBj], oi[kBj];
 #pragma unroll
-    for (int c = 0; c < 2 * kBj; ++c) {
+    for (int c = 0; c < kBj; ++c) {
       orr[c] = c < w ? Wm.r(row, colof(c)) : 0.0;
       oi[c] = (C && c < w) ? Wm.m(row, colof(c)) : 0.0;
     }
     for (int c = 0; c < w; ++c) {
       double sr = 0.0, si = 0.0;
 #pragma unroll
-      for (int c2 = 0; c2 < 2 * kBj; ++c2) {
+      for (int c2 = 0; c2 < kBj; ++c2) {
         if (c2 >= w) break;
         const double vr = Vr[c * w + c2], vi = Vi[c * w + c2];  // V[c2, c]
         sr += orr[c2] * vr - (C ? oi[c2] * vi : 0.0);
@@ -1057,6 +1062,203 @@ __global__ __launch_bounds__(kThreads) void svd_block_round_kernel(const SvdTask
     }
   }
   if (tid == 0) rotated[sidx] = 1.0;
+}
+
+// A barrier that waits for this wave's LDS accesses only: global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The rounds across blocks (round >= 0): wave a keeps column a of block I in
+// registers through all kBj sub-rounds and meets column (a + sub) mod kBj of
+// block J, which is in LDS, so a sub-round reads one column and writes one
+// where columns of both blocks in LDS cost two of each.  Latency bounds it:
+// every launch waits for the one before, so the sector is found by one wave
+// read, the columns of A and Wm are requested together before the first
+// wait, and for columns of at most 64 NQ rows (zero beyond r) no sub-round
+// has a branch on the row.  Mean launch: real, r up to 256: 13.0 us against
+// 20 with both blocks in LDS and the quotient form of the rotation; complex,
+// r up to 128 (Hubbard L = 20, D = 192, 4 vectors): 15.5 us against 20.
+template <bool C, int NQ>
+__global__ __launch_bounds__(kThreads) void svd_block_across_kernel(const SvdTask* __restrict__ tasks, int ntasks,
+                                                                    const int* __restrict__ pair_base, int round,
+                                                                    double* __restrict__ W, int64_t w_plane,
+                                                                    double* __restrict__ rotated) {
+  constexpr int kRows = 64 * NQ, kPairs = 2 * kBj;
+  extern __shared__ double blk_lds[];  // block J: kBj columns of kRows, per plane
+  double* const Lr = blk_lds;
+  double* const Li = blk_lds + kBj * kRows;
+  __shared__ double Vr[kPairs * kPairs], Vi[kPairs * kPairs];  // column c at c * kPairs
+  __shared__ int any;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // sector of this workgroup: pair_base is ascending, pair_base[0] = 0
+  int s = 0;
+  for (int n = ntasks; n > 1;) {
+    const int step = (n + 63) >> 6, i = lane * step;
+    const bool ok = i < n && pair_base[s + (i < n ? i : 0)] <= (int)blockIdx.x;
+    const int c = __popcll(__ballot(ok)) - 1;
+    s += c * step;
+    n = min(step, n - c * step);
+  }
+  s = __builtin_amdgcn_readfirstlane(s);
+  const SvdTask t = tasks[s];
+  const int q = (int)blockIdx.x - pair_base[s];
+  const int p = t.m < t.n ? t.n : t.m, r = t.m < t.n ? t.m : t.n;
+  const int nb = (r + kBj - 1) / kBj, nbb = nb + (nb & 1);
+  if (r > kRows || round >= nbb - 1 || q >= nbb / 2) return;
+  int I = (round + q) % (nbb - 1);
+  int J = q == 0 ? nbb - 1 : (round + nbb - 1 - q) % (nbb - 1);
+  if (I > J) {
+    const int x = I;
+    I = J;
+    J = x;
+  }
+  if (J >= nb) return;  // the bye of an odd block count
+  const int i0 = I * kBj, j0 = J * kBj, w = kBj + min(kBj, r - j0);  // J > I: block I is whole
+  const int64_t o_wm = (int64_t)p * r, o_a = 2 * (int64_t)p * r + (int64_t)r * r;
+  Mat<C> Wm{W + t.w_off + o_wm, W + t.w_off + o_wm + w_plane, r};
+  Mat<C> A{W + t.w_off + o_a, W + t.w_off + o_a + w_plane, r};
+  // column c of the pair's 2 kBj; those past the sector read its last one
+  auto colof = [&](int c) { return c < kBj ? i0 + c : min(j0 + c - kBj, r - 1); };
+  const bool has = kBj + wave < w;
+  double xr[NQ], xi[NQ];
+  {
+    double jr[NQ], ji[NQ];
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      const int row = min(lane + 64 * k, r - 1);
+      xr[k] = A.r(row, i0 + wave);
+      jr[k] = A.r(row, colof(kBj + wave));
+      if (C) {
+        xi[k] = A.m(row, i0 + wave);
+        ji[k] = A.m(row, colof(kBj + wave));
+      }
+    }
+    if (tid < kPairs * kPairs) {
+      Vr[tid] = tid % kPairs == tid / kPairs ? 1.0 : 0.0;
+      Vi[tid] = 0.0;
+    }
+    if (tid == 0) any = 0;
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      const bool in = lane + 64 * k < r;
+      xr[k] = in ? xr[k] : 0.0;
+      Lr[wave * kRows + lane + 64 * k] = in && has ? jr[k] : 0.0;
+      if (C) {
+        xi[k] = in ? xi[k] : 0.0;
+        Li[wave * kRows + lane + 64 * k] = in && has ? ji[k] : 0.0;
+      }
+    }
+  }
+  // this thread's row of Wm's columns: kThreads / kRows threads share a row and
+  // write kNc columns each
+  constexpr int kNc = kPairs * kRows / kThreads;
+  const int wrow = tid % kRows, c_lo = __builtin_amdgcn_readfirstlane(tid / kRows) * kNc;
+  double wr[kPairs], wi[kPairs];
+#pragma unroll
+  for (int c = 0; c < kPairs; ++c) {
+    const double re = Wm.r(min(wrow, r - 1), colof(c)), im = C ? Wm.m(min(wrow, r - 1), colof(c)) : 0.0;
+    wr[c] = c < w ? re : 0.0;
+    wi[c] = c < w ? im : 0.0;
+  }
+  lds_barrier();
+  const double tol = sqrt((double)r) * DBL_EPSILON;
+  for (int sub = 0; sub < kBj; ++sub) {
+    const int j = (wave + sub) % kBj;
+    double* const yjr = Lr + j * kRows + lane;
+    double* const yji = Li + j * kRows + lane;
+    double yr[NQ], yi[NQ], a = 0.0, bb = 0.0, gr = 0.0, gi = 0.0;
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      yr[k] = yjr[64 * k];
+      if (C) yi[k] = yji[64 * k];
+    }
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      a += xr[k] * xr[k];
+      bb += yr[k] * yr[k];
+      gr += xr[k] * yr[k];
+      if (C) {
+        a += xi[k] * xi[k];
+        bb += yi[k] * yi[k];
+        gr += xi[k] * yi[k];
+        gi += xr[k] * yi[k] - xi[k] * yr[k];
+      }
+    }
+    a = wave_sum(a);
+    bb = wave_sum(bb);
+    gr = wave_sum(gr);
+    if (C) gi = wave_sum(gi);
+    double c, sn, er, ei;
+    if (jacobi_rotation<C>(a, bb, gr, gi, tol, c, sn, er, ei)) {
+      // x' = c x - s conj(e) y, y' = s e x + c y (as rotate_cols), on the columns and on V
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) {
+        if (C) {
+          const double ujr = er * yr[k] + ei * yi[k], uji = er * yi[k] - ei * yr[k];
+          const double uir = er * xr[k] - ei * xi[k], uii = er * xi[k] + ei * xr[k];
+          xr[k] = c * xr[k] - sn * ujr;
+          xi[k] = c * xi[k] - sn * uji;
+          yjr[64 * k] = sn * uir + c * yr[k];
+          yji[64 * k] = sn * uii + c * yi[k];
+        } else {
+          const double x0 = xr[k];
+          xr[k] = c * x0 - sn * er * yr[k];
+          yjr[64 * k] = sn * er * x0 + c * yr[k];
+        }
+      }
+      if (lane < kPairs) {
+        const int ci = wave * kPairs + lane, cj = (kBj + j) * kPairs + lane;
+        const double vir = Vr[ci], vjr = Vr[cj];
+        if (C) {
+          const double vii = Vi[ci], vji = Vi[cj];
+          Vr[ci] = c * vir - sn * (er * vjr + ei * vji);
+          Vi[ci] = c * vii - sn * (er * vji - ei * vjr);
+          Vr[cj] = sn * (er * vir - ei * vii) + c * vjr;
+          Vi[cj] = sn * (er * vii + ei * vir) + c * vji;
+        } else {
+          Vr[ci] = c * vir - sn * er * vjr;
+          Vr[cj] = sn * er * vir + c * vjr;
+        }
+      }
+      if (lane == 0) any = 1;
+    }
+    lds_barrier();
+  }
+  if (!any) return;  // uniform: read after the last barrier; nothing changed
+  // every thread's row of Wm has arrived before the threads that share it write
+#pragma unroll
+  for (int c = 0; c < kPairs; ++c) {
+    asm volatile("" : "+v"(wr[c]));
+    if (C) asm volatile("" : "+v"(wi[c]));
+  }
+  lds_barrier();
+  // columns back to A; Wm[:, cols] <- Wm[:, cols] V
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int row = lane + 64 * k;
+    if (row >= r) continue;
+    A.r(row, i0 + wave) = xr[k];
+    if (C) A.m(row, i0 + wave) = xi[k];
+    if (has) {
+      A.r(row, j0 + wave) = Lr[wave * kRows + row];
+      if (C) A.m(row, j0 + wave) = Li[wave * kRows + row];
+    }
+  }
+  if (wrow < r)
+    for (int c = c_lo; c < min(w, c_lo + kNc); ++c) {
+      double sr = 0.0, si = 0.0;
+#pragma unroll
+      for (int c2 = 0; c2 < kPairs; ++c2) {
+        const double vr = Vr[c * kPairs + c2], vi = C ? Vi[c * kPairs + c2] : 0.0;
+        sr += wr[c2] * vr - (C ? wi[c2] * vi : 0.0);
+        if (C) si += wr[c2] * vi + wi[c2] * vr;
+      }
+      Wm.r(wrow, colof(c)) = sr;
+      if (C) Wm.m(wrow, colof(c)) = si;
+    }
+  if (tid == 0) rotated[s] = 1.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1089,7 +1291,7 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
   __shared__ double hv[3];
   // X of a small sector, or the general path's reflection vector; 64 KB: two
   // workgroups per CU
-  constexpr int kCap = 8192 - 6 * kSmallCols;
+  constexpr int kCap = kQrLds;
   __shared__ double buf[kCap];
   __shared__ double scal[6][kSmallCols];
   static_assert(2 * kVecRows <= kCap, "the reflection vector fits");
@@ -1099,7 +1301,7 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
   if (m <= 0 || n <= 0) return;
   const int p = right ? n : m, r = right ? m : n, k = p < r ? p : r;
   const int tid = threadIdx.x;
-  if (phases == kPhAll && small_fits(p, r, C, kCap)) {
+  if (phases == kPhAll && qr_in_lds(m, n, right, C)) {
     const SmallQr<C> f{buf, buf + p * r, scal, p, r, k};
     for (int e = tid; e < p * r; e += kQrThreads) {
       // neighbouring threads read neighbouring elements of M
@@ -1421,30 +1623,47 @@ hipError_t launch_svd_phase(int cplx, int phases, const SvdTask* tasks, int ntas
   return hipGetLastError();
 }
 
+namespace {
+// NQ: the smallest that holds the launch's longest column (an unused column
+// segment costs LDS traffic and registers, a branch on it a wait)
+template <bool C>
+hipError_t block_round(const SvdTask* tasks, int ntasks, const int* pair_base, int npairs, int round, double* W,
+                       int64_t w_plane, double* rotated, int rmax, hipStream_t st) {
+  static bool attr = false;  // the dynamic LDS limit, raised once
+  constexpr size_t kCol = sizeof(double) * (C ? 2 : 1) * kBj;  // bytes of a block's row
+  if (!attr) {
+    const void* k[2] = {(const void*)svd_block_inner_kernel<C>, (const void*)svd_block_across_kernel<C, 8>};
+    for (const void* f : k) {
+      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kCol * kBjMaxR));
+      if (e != hipSuccess) return e;
+    }
+    attr = true;
+  }
+  if (round < 0)
+    svd_block_inner_kernel<C><<<2 * npairs, kThreads, kCol * rmax, st>>>(tasks, ntasks, pair_base, W, w_plane, rotated,
+                                                                         rmax);
+  else if (rmax <= 64)
+    svd_block_across_kernel<C, 1><<<npairs, kThreads, kCol * 64, st>>>(tasks, ntasks, pair_base, round, W, w_plane,
+                                                                       rotated);
+  else if (rmax <= 128)
+    svd_block_across_kernel<C, 2><<<npairs, kThreads, kCol * 128, st>>>(tasks, ntasks, pair_base, round, W, w_plane,
+                                                                        rotated);
+  else if (rmax <= 256)
+    svd_block_across_kernel<C, 4><<<npairs, kThreads, kCol * 256, st>>>(tasks, ntasks, pair_base, round, W, w_plane,
+                                                                        rotated);
+  else
+    svd_block_across_kernel<C, 8><<<npairs, kThreads, kCol * 512, st>>>(tasks, ntasks, pair_base, round, W, w_plane,
+                                                                        rotated);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_svd_block_round(int cplx, const SvdTask* tasks, int ntasks, const int* pair_base, int npairs,
                                   int round, double* W, int64_t w_plane, double* rotated, int rmax, hipStream_t st) {
   if (ntasks <= 0 || npairs <= 0) return hipSuccess;
   if (rmax < 1 || rmax > kBjMaxR) return hipErrorInvalidValue;
-  static bool attr[2] = {false, false};  // the dynamic LDS limit, raised once per kernel
-  const size_t lds = sizeof(double) * (cplx ? 2 : 1) * 2 * kBj * (size_t)rmax;
-  const size_t lds_max = sizeof(double) * 2 * 2 * kBj * (size_t)kBjMaxR;
-  if (!attr[cplx ? 1 : 0]) {
-    const hipError_t e =
-        cplx ? hipFuncSetAttribute((const void*)svd_block_round_kernel<true>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max)
-             : hipFuncSetAttribute((const void*)svd_block_round_kernel<false>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(lds_max / 2));
-    if (e != hipSuccess) return e;
-    attr[cplx ? 1 : 0] = true;
-  }
-  const int grid = round < 0 ? 2 * npairs : npairs;
-  if (cplx)
-    svd_block_round_kernel<true><<<grid, kThreads, lds, st>>>(tasks, ntasks, pair_base, round, W, w_plane, rotated,
-                                                              rmax);
-  else
-    svd_block_round_kernel<false><<<grid, kThreads, lds, st>>>(tasks, ntasks, pair_base, round, W, w_plane, rotated,
-                                                               rmax);
-  return hipGetLastError();
+  if (cplx) return block_round<true>(tasks, ntasks, pair_base, npairs, round, W, w_plane, rotated, rmax, st);
+  return block_round<false>(tasks, ntasks, pair_base, npairs, round, W, w_plane, rotated, rmax, st);
 }
 
 hipError_t launch_house_panels(int cplx, int layout, const SvdTask* tasks, int ntasks, const int* col_base,

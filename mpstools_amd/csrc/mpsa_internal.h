@@ -150,6 +150,12 @@ struct SvdTask {
 hipError_t launch_svd_batched(int cplx, const SvdTask* tasks, int ntasks, const double* M, int64_t m_plane,
                               double* U, int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W,
                               int64_t w_plane, hipStream_t st);
+// Sectors that launch_qr_batched factorises in one workgroup's LDS: at most 512
+// rows and 64 columns of X (M, or M^H when right), kQrLds doubles.
+constexpr int kQrLds = 7808;
+constexpr bool qr_in_lds(int64_t m, int64_t n, int right, bool cplx) {
+  return (right ? n : m) <= 512 && (right ? m : n) <= 64 && m * n * (cplx ? 2 : 1) <= kQrLds;
+}
 // The same SVD in phases for large sectors (the kPh* bits below), several
 // workgroups per sector for the reflections, the sweeps and the
 // back-transform: the sweeps are launch_svd_block_round launches (one per

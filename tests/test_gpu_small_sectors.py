@@ -66,3 +66,36 @@ def test_small_complex_factorisations(gpu, L, D, seed):
         for blocks in by.values():
             X = np.hstack(blocks)
             assert np.max(np.abs(X @ X.conj().T - np.eye(X.shape[0]))) <= 1e-12
+
+
+@pytest.mark.parametrize("dl,dr,scale", [(16, 17, 1.0), (17, 17, 1.0), (20, 90, 1.0), (33, 32, 1.0), (63, 64, 1.0),
+                                         (65, 65, 1.0), (128, 140, 1.0), (129, 130, 1.0), (21, 30, 1e70),
+                                         (7, 9, 1e70)])
+def test_block_rounds_at_their_edges(gpu, dl, dr, scale):
+    """Sectors of several column blocks: a whole last block and one of 2 to 6
+    columns, odd and even block counts, either side of 128 and 256 rows (the
+    shares of the vectors' update); norms near 1e140, where the rotation's
+    squares leave the doubles' range.  Singular values 1 .. 2^-4 (relative
+    error n eps < 1e-13 each), state rebuilt within 1e-12 relative."""
+    torch = gpu
+    print("[case] block rounds", 2 * dl, 2 * dr, scale, flush=True)
+    rng = np.random.default_rng(31 * dl + dr)
+    m, n = 2 * dl, 2 * dr
+    k = min(m, n)
+    U = np.linalg.qr(rng.standard_normal((m, k)))[0]
+    V = np.linalg.qr(rng.standard_normal((n, k)))[0]
+    sv = 2.0 ** (-4.0 * np.arange(k) / k)
+    M = (U * (sv * scale)) @ V.T
+    psi = Blocks(2)
+    for s1 in range(2):
+        for s2 in range(2):
+            psi[(0, 0, s1, s2)] = M[s1 * dl:(s1 + 1) * dl, s2 * dr:(s2 + 1) * dr]
+    t = native.Table.from_blocks(psi)
+    out = native.split(t, torch.from_numpy(t.pack(psi)).cuda(), [0, 0], [0, 0], direction=1, chimax=10 ** 6)
+    got = np.asarray(out["lam"][0])
+    got = got / np.linalg.norm(got)
+    assert got.shape == (k,) and np.max(np.abs(got / (sv / np.linalg.norm(sv)) - 1.0)) <= 1e-13
+    two = twosite(out["left"][0].unpack(out["left"][1].cpu().numpy()),
+                  out["right"][0].unpack(out["right"][1].cpu().numpy()))
+    ratio = np.vdot(two[(0, 0, 0, 0)], psi[(0, 0, 0, 0)]) / np.vdot(two[(0, 0, 0, 0)], two[(0, 0, 0, 0)])
+    assert max(np.max(np.abs(two[key] * (ratio / scale) - psi[key] / scale)) for key in psi.keys()) <= 1e-12
