@@ -266,6 +266,7 @@ struct mpsa_cheb {
   // sectors with min(m, n) at least this (and at most kSvdBlockMaxR) take the
   // blocked Jacobi SVD, several workgroups per sector; 0: never
   int64_t block_min_r = MPSA_BLOCK_JACOBI_MIN;
+  bool block_set = false;  // block_min_r is the caller's
   // host time (seconds): plan builds, output-key queries, waits on the stream
   double t_plan = 0.0, t_keys = 0.0, t_sync = 0.0;
   double t_heff = 0.0, t_env = 0.0, t_prep = 0.0;  // host seconds in heff1, env_layer, prepare_site
@@ -760,8 +761,10 @@ void prepare_site(Eng& E, DMps& M, int site, bool left, bool keep_lambda) {
     if (!S.big) tw += use_qr ? align64(S.m * S.n + qp * S.k + S.k) : align64(svd_workspace(S.m, S.n));
   }
   const int pl = E.planes;
-  Buf Mb(E.pool, pl * tm, E.st), Ub(E.pool, pl * tu, E.st), Vb(E.pool, pl * tv, E.st), Sb(E.pool, ts, E.st),
-      Wb(E.pool, pl * tw, E.st, false);
+  // none is cleared: the blocks of a sector tile its matrix, and the
+  // factorisations write every element of their outputs
+  Buf Mb(E.pool, pl * tm, E.st, false), Ub(E.pool, pl * tu, E.st, false), Vb(E.pool, pl * tv, E.st, false),
+      Sb(E.pool, ts, E.st, false), Wb(E.pool, pl * tw, E.st, false);
   // gather
   std::vector<Copy2D> g;
   const int64_t xoff_plane = X.total;
@@ -824,7 +827,12 @@ void prepare_site(Eng& E, DMps& M, int site, bool left, bool keep_lambda) {
     std::vector<SvdTask> rest;
     for (const SvdTask& t : tasks) {
       const int64_t r = std::min(t.m, t.n), p = std::max(t.m, t.n);
-      const bool ok = r >= E.block_min_r && p <= kVecRowsMax && (use_qr || r <= kSvdBlockMaxR);
+      // without a limit of the caller's, the QR of a sector that one workgroup
+      // holds in LDS stays with one: no launches between its panels (three
+      // moments, Hubbard L = 20, D = 192, 4 vectors, complex: the QR kernels
+      // take 85 ms a call so, 98 ms in panels over several workgroups)
+      const bool one = !E.block_set && use_qr && qr_in_lds(t.m, t.n, left ? 0 : 1, pl == 2);
+      const bool ok = r >= E.block_min_r && !one && p <= kVecRowsMax && (use_qr || r <= kSvdBlockMaxR);
       (ok ? blocked : rest).push_back(t);
     }
     tasks.swap(rest);
@@ -1866,6 +1874,7 @@ int mpsa_cheb_set_block_jacobi(mpsa_cheb* E, int r) {
     return MPSA_EINVAL;
   }
   E->block_min_r = r;
+  E->block_set = true;
   return MPSA_OK;
 }
 
