@@ -93,7 +93,7 @@ constexpr double kDmTail = 1e-4;
 // workgroups share a sector) go to the library's batched one-sided Jacobi SVD
 // (mpsa_factor.hip), all of them in the same launches; larger ones to
 // rocSOLVER's gesvdj, one call and one wait each.  The t-V D = 512 bond (16
-// sectors of up to 160 x 160): 166 ms by gesvdj, 7.6 ms here.
+// sectors of up to 160 x 160): 166 ms by gesvdj, 4.8 ms here.
 constexpr int64_t kOwnBlockR = 32, kOwnMaxR = kSvdBlockMaxR, kOwnMaxP = 4096;
 bool own_svd(int64_t m, int64_t n) {
   const int64_t r = std::min(m, n), p = std::max(m, n);
@@ -361,7 +361,8 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
       if (!blocked.empty()) {
         flags.alloc(blocked.size());
         hchk(launch_fill(flags.p, (int64_t)blocked.size(), 0.0, st), "split: flags");
-        svd_blocked_run(dev, false, blocked, M.p, 0, U.p, 0, V.p, 0, Sg.p, Wk.p, 0, flags.p, st);
+        if (!svd_blocked_run(dev, false, blocked, M.p, 0, U.p, 0, V.p, 0, Sg.p, Wk.p, 0, flags.p, st))
+          throw SErr(MPSA_EINVAL, "split: sector SVD did not converge");
       }
     }
     const double one = 1.0, zero = 0.0;
@@ -507,6 +508,14 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
     std::vector<double> sv((size_t)std::max<int64_t>(tot_S, 1));
     if (tot_S) hchk(hipMemcpyAsync(sv.data(), Sg.p, sizeof(double) * tot_S, hipMemcpyDeviceToHost, st), "split: S");
     hchk(hipStreamSynchronize(st), "split: sync");
+    // the batched SVD's sweeps end at once on columns of NaN, which gesvdj
+    // reports as not converged
+    for (auto& kv : secs) {
+      const Sector& S = kv.second;
+      if (dm_route(S) || !own_svd(S.m, S.n)) continue;
+      for (int64_t i = 0; i < S.k; ++i)
+        if (!std::isfinite(sv[(size_t)(S.off_S + i)])) throw SErr(MPSA_EINVAL, "split: sector SVD did not converge");
+    }
 
     // global truncation over all sectors (src/BlockTensor.hpp:85-136, 234-276):
     // multimap<sigma, qc> filled sector by sector in key order, visited from

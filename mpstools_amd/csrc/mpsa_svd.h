@@ -28,9 +28,10 @@ inline int house_table(const std::vector<SvdTask>& ts, int layout, std::vector<i
 //                                           valid until the next wait after its use
 //   void check(hipError_t, const char*)     throws on an error
 //   void wait()                             drains the stream
-// flags: big.size() doubles of device memory, zero.
+// flags: big.size() doubles of device memory, zero.  False when a sector still
+// rotates after 60 sweeps.
 template <class Dev>
-void svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const double* M, int64_t m_plane, double* U,
+bool svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const double* M, int64_t m_plane, double* U,
                      int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W, int64_t w_plane,
                      double* flags, hipStream_t st) {
   const int nb = (int)big.size();
@@ -75,6 +76,7 @@ void svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const
   phase(kPhBackInit, "sector SVD back-transform");
   dev.check(launch_house_apply(cplx, 0, t, nb, dh, hbase.back(), W, w_plane, st), "sector SVD back-transform");
   phase(kPhOut, "sector SVD outputs");
+  return act.empty();
 }
 
 }  // namespace mpsa

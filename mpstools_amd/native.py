@@ -737,7 +737,8 @@ class Cheb:
         """Sectors with min(m, n) >= r_min and max(m, n) <= 1024 are
         factorised by several workgroups each (Householder panels, Q
         formation, and for SVD steps with min(m, n) <= 512 the block Jacobi
-        rounds); 0: one workgroup per sector; default 32."""
+        rounds); 0: one workgroup per sector; default 32, but QR sectors that
+        fit one workgroup's LDS stay there until this is called."""
         _check(lib().mpsa_cheb_set_block_jacobi(self.h, int(r_min)))
 
     def factor_log(self, cap):

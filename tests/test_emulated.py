@@ -323,7 +323,7 @@ def test_emulated_split_matches_oracle(lib, oracle, model, L, N, D, seed, dense,
     density-matrix route built here for sectors with min(m, n) >= 64: the
     dense centre bond is one 96 x 96 sector of rank 48, the dense bond at
     sites 5, 6 of L = 16 one wide 64 x 128 sector.  Untruncated
-    (chimax = 10^6) they go to gesvdj, which reveals the rank; count-limited
+    (chimax = 10^6) they go to the Jacobi SVD, which reveals the rank; count-limited
     (chimax = 40, 50, 60) to the eigendecomposition of M M^T, where
     chimax = 60 is above the rank (48) and needs the route's rank guard.  Bars: singular
     values within 1e-12 relative or 100 eps lambda_max (LAPACK on both sides
