@@ -70,7 +70,7 @@ def test_small_complex_factorisations(gpu, L, D, seed):
 
 @pytest.mark.parametrize("dl,dr,scale", [(16, 17, 1.0), (17, 17, 1.0), (20, 90, 1.0), (33, 32, 1.0), (63, 64, 1.0),
                                          (65, 65, 1.0), (128, 140, 1.0), (129, 130, 1.0), (21, 30, 1e70),
-                                         (7, 9, 1e70)])
+                                         (7, 9, 1e70), (17, 512, 1.0), (512, 19, 1.0)])
 def test_block_rounds_at_their_edges(gpu, dl, dr, scale):
     """Sectors of several column blocks: a whole last block and one of 2 to 6
     columns, odd and even block counts, either side of 128 and 256 rows (the
