@@ -511,8 +511,9 @@ int mpsa_cheb_set_big_sector(mpsa_cheb* engine, int k);
  * are factorised by several workgroups each: the Householder reflections in
  * panels of 8 columns, Q and the SVD's back-transform column by column, and
  * (SVD steps, r <= 512) the blocked Jacobi sweeps, one launch per round of
- * the block tournament and one host wait per sweep.  r_min = 0 keeps every
- * sector in the one-workgroup kernels.  Same factorisation either way (no
+ * the block tournament and one host wait per sweep.  Without a call, the QR
+ * of a sector that fits one workgroup's LDS stays in one.  r_min = 0 keeps
+ * every sector in the one-workgroup kernels.  Same factorisation either way (no
  * counterpart in the reference: a scheduling choice). */
 int mpsa_cheb_set_block_jacobi(mpsa_cheb* engine, int r_min);
 /* Sector-shape log of the canonicalisation launches (a profiling aid with no

@@ -93,7 +93,7 @@ constexpr double kDmTail = 1e-4;
 // workgroups share a sector) go to the library's batched one-sided Jacobi SVD
 // (mpsa_factor.hip), all of them in the same launches; larger ones to
 // rocSOLVER's gesvdj, one call and one wait each.  The t-V D = 512 bond (16
-// sectors of up to 160 x 160): 166 ms by gesvdj, 4.8 ms here.
+// sectors of up to 160 x 160): 166 ms by gesvdj, 4.7 ms here.
 constexpr int64_t kOwnBlockR = 32, kOwnMaxR = kSvdBlockMaxR, kOwnMaxP = 4096;
 bool own_svd(int64_t m, int64_t n) {
   const int64_t r = std::min(m, n), p = std::max(m, n);
