@@ -757,8 +757,7 @@ void prepare_site(Eng& E, DMps& M, int site, bool left, bool keep_lambda) {
     S.so = ts;
     ts += S.k;
     S.wo = tw;
-    const int64_t qp = left ? S.m : S.n;  // rows of the factorised X = M or M^H
-    if (!S.big) tw += use_qr ? align64(S.m * S.n + qp * S.k + S.k) : align64(svd_workspace(S.m, S.n));
+    if (!S.big) tw += align64(use_qr ? qr_workspace(S.m, S.n, left ? 0 : 1) : svd_workspace(S.m, S.n));
   }
   const int pl = E.planes;
   // none is cleared: the blocks of a sector tile its matrix, and the
@@ -979,6 +978,9 @@ void prepare_site(Eng& E, DMps& M, int site, bool left, bool keep_lambda) {
     std::vector<double> h((size_t)std::max<int64_t>(ts, 1));
     if (ts) hchk(hipMemcpyAsync(h.data(), Sb.p, sizeof(double) * (size_t)ts, hipMemcpyDeviceToHost, E.st), "cheb: S");
     E.sync();
+    // NaN: a sector without factors (mpsa_factor.hip)
+    for (int64_t i = 0; i < ts; ++i)
+      if (!std::isfinite(h[(size_t)i])) throw HErr(MPSA_EINVAL, "cheb: the SVD of a sector did not converge");
     auto& L = M.lam[(size_t)(left ? site : site - 1)];
     L.clear();
     for (auto& kv : secs) L[kv.first].assign(h.begin() + kv.second.so, h.begin() + kv.second.so + kv.second.k);

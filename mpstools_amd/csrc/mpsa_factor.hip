@@ -23,6 +23,8 @@
 // Singular vectors of exactly zero singular values (on the Z side; Q Wm is
 // orthonormal by construction) are completed to an orthonormal basis
 // (Gram-Schmidt of unit vectors, twice), as a LAPACK thin SVD returns them.
+// A sector whose matrix holds a value that is not finite has NaN in every
+// output.
 // Real data: FixPhase makes the first largest-|.| entry of every row of
 // V^dagger positive (the column of U flips with it).
 //
@@ -61,6 +63,30 @@ __device__ __forceinline__ double wave_sum(double x) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(x), 63);
   const int hi = __builtin_amdgcn_readlane(__double2hiint(x), 63);
   return __hiloint2double(hi, lo);
+}
+
+// High word of |x|: ordered as the values are, kNotFinite and above for Inf
+// and NaN.  The loads of a sector collect its maximum, since NaN fails every
+// comparison that the reflections and rotations make and would be left out.
+constexpr int kNotFinite = 0x7ff00000;
+__device__ __forceinline__ int magnitude(double x) { return __double2hiint(x) & 0x7fffffff; }
+// Maximum of x over the workgroup, in every thread; red: one int per wave
+// (LDS).  All LDS written before is visible after.
+template <int NT>
+__device__ __forceinline__ int group_max(int x, int* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x = max(x, __shfl_xor(x, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) x = max(x, red[w]);
+  return x;
+}
+// What a sector's values are multiplied by at the outputs: NaN where its
+// matrix holds a value that is not finite, so that no caller takes the
+// factors for a result.
+__device__ __forceinline__ double sector_scale(int mx) {
+  return mx >= kNotFinite ? __longlong_as_double(0x7ff8000000000000ll) : 1.0;
 }
 
 // Column j of a p-row matrix with leading dimension ld, planar complex.
@@ -338,12 +364,11 @@ struct SmallQr {
   int p, r, k;
   __device__ __forceinline__ double& re(int i, int j) const { return xr[i + j * p]; }
   __device__ __forceinline__ double& im(int i, int j) const { return xi[i + j * p]; }
-  // X = Q R in place; starts and ends with a barrier
+  // X = Q R in place, X complete behind a barrier; ends with one
   template <int NT>
   __device__ __forceinline__ void factor() const {
     constexpr int NW = NT / 64;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    __syncthreads();
     if (wave == 0) {
       double a = 0.0;
       for (int i = lane; i < p; i += 64) {
@@ -543,7 +568,7 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
                                                               int64_t w_plane, int max_sweeps, int phases) {
   __shared__ double sig[kSvdMaxR];
   __shared__ int rank[kSvdMaxR];
-  __shared__ int rotated;
+  __shared__ int rotated, mxw[kWaves];
   __shared__ double red[kWaves], redc[kWaves];
   __shared__ double hv[3];
   // X, A and Wm of a small sector, or the general path's reflection vector
@@ -565,27 +590,34 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
   // factor are closer to orthogonal than its columns).  The p-side singular
   // vectors Q Wm are orthonormal by construction; the r-side ones are the
   // rotated columns of A divided by sigma.  Workspace: X (p x r), Wm (r x r),
-  // the reflection vectors (p x r), A (r x r), betas (r).
+  // the reflection vectors (p x r), A (r x r), betas (r), the scale.
   Mat<C> X{W + t.w_off, W + t.w_off + w_plane, p};
   Mat<C> Wm{W + t.w_off + (int64_t)p * r, W + t.w_off + (int64_t)p * r + w_plane, r};
   const int64_t o_hv = (int64_t)p * r + (int64_t)r * r, o_a = 2 * (int64_t)p * r + (int64_t)r * r;
   Mat<C> Hv{W + t.w_off + o_hv, W + t.w_off + o_hv + w_plane, p};
   Mat<C> A{W + t.w_off + o_a, W + t.w_off + o_a + w_plane, r};
   double* const beta = W + t.w_off + o_a + (int64_t)r * r;
+  double* const state = beta + r;  // the sector's scale, for the phases
+  double scale = 1.0;
   // A small sector: reflections, sweeps and back-transform in LDS, A and
   // X = Q [Wm; 0] then in the workspace for the outputs below.  (A sweep of 30
   // columns is 30 rounds, each of which waits for memory on the general path.)
-  if (phases == kPhAll && small_fits(p, r, C, kCap - (C ? 4 : 2) * r * r)) {
+  const bool small = phases == kPhAll && small_fits(p, r, C, kCap - (C ? 4 : 2) * r * r);
+  if (small) {
     constexpr int NP = C ? 2 : 1;
     double* const la = buf + NP * p * r;
     double* const lw = la + NP * r * r;
     const SmallQr<C> f{buf, buf + p * r, scal, p, r, r};
+    int mx = 0;
     for (int e = tid; e < p * r; e += kThreads) {
       const int i = wide ? e / r : e % p, j = wide ? e % r : e / p;
       const int64_t src = t.a_off + (wide ? j + (int64_t)i * t.lda : i + (int64_t)j * t.lda);
-      f.re(i, j) = M[src];
-      if (C) f.im(i, j) = wide ? -M[m_plane + src] : M[m_plane + src];
+      const double x = M[src], y = C ? M[m_plane + src] : 0.0;
+      mx = max(mx, max(magnitude(x), magnitude(y)));
+      f.re(i, j) = x;
+      if (C) f.im(i, j) = wide ? -y : y;
     }
+    scale = sector_scale(group_max<kThreads>(mx, mxw));
     f.template factor<kThreads>();
     for (int e = tid; e < r * r; e += kThreads) {  // A = R^H, Wm = I
       const int i = e % r, j = e / r;
@@ -627,13 +659,19 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
   // and the outputs, each phase reading what the previous left in the workspace
   // X = M or M^H
   if (phases & kPhLoad) {
+    int mx = 0;
     for (int64_t e = tid; e < (int64_t)p * r; e += kThreads) {
       const int i = (int)(e % p), j = (int)(e / p);
-      const int64_t src = wide ? (j + (int64_t)i * t.lda) : (i + (int64_t)j * t.lda);
-      X.r(i, j) = M[t.a_off + src];
-      if (C) X.m(i, j) = wide ? -M[t.a_off + m_plane + src] : M[t.a_off + m_plane + src];
+      const int64_t src = t.a_off + (wide ? (j + (int64_t)i * t.lda) : (i + (int64_t)j * t.lda));
+      const double x = M[src], y = C ? M[m_plane + src] : 0.0;
+      mx = max(mx, max(magnitude(x), magnitude(y)));
+      X.r(i, j) = x;
+      if (C) X.m(i, j) = wide ? -y : y;
     }
-    __syncthreads();
+    scale = sector_scale(group_max<kThreads>(mx, mxw));
+    if (tid == 0) *state = scale;
+  } else if (!small) {
+    scale = *state;
   }
   if (phases & kPhReflect) house_reflect<C, kThreads>(X, Hv, beta, p, r, red, hv, vl);
   // A = R^H (lower triangular), Wm = identity
@@ -743,9 +781,23 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
       }
     }
     a = wave_sum(a);
-    if (lane == 0) sig[j] = sqrt(a);
+    a = sqrt(a);
+    if (lane == 0) sig[j] = a;
+    if (!(a <= DBL_MAX)) scale = a;
   }
-  __syncthreads();
+  if (__syncthreads_or(!(scale <= DBL_MAX))) {  // no factors: every output NaN
+    const double none = sector_scale(kNotFinite);
+    for (int i = tid; i < k; i += kThreads) S[t.s_off + i] = none;
+    for (int64_t e = tid; e < (int64_t)m * k; e += kThreads) {
+      U[t.u_off + e] = none;
+      if (C) U[t.u_off + u_plane + e] = none;
+    }
+    for (int64_t e = tid; e < (int64_t)k * n; e += kThreads) {
+      Vt[t.vt_off + e] = none;
+      if (C) Vt[t.vt_off + vt_plane + e] = none;
+    }
+    return;
+  }
   for (int j = tid; j < r; j += kThreads) {
     int rk = 0;
     const double sj = sig[j];
@@ -1270,7 +1322,9 @@ __global__ __launch_bounds__(kThreads) void svd_block_across_kernel(const SvdTas
 // |x|) zeroes column j below the diagonal, applied to columns j+1.. one wave
 // per column; then Q = H_0 ... H_{k-1} [I; 0] is accumulated backwards
 // (columns j.. of the partial product, as LAPACK's xORGQR does).
-// Workspace per task: p r (X) + p k (vectors) + k (betas) elements per plane.
+// Workspace per task (qr_workspace): X (p r), the vectors (p k), the betas (k)
+// and the scale, per plane.  A matrix with a value that is not finite gives an
+// R of NaN.
 constexpr int kQrThreads = 512;
 constexpr int kQrWaves = kQrThreads / 64;
 
@@ -1283,8 +1337,8 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
                                                                     int64_t w_plane, int phases) {
   __shared__ double red[kQrWaves];
   __shared__ double hv[3];
-  // X of a small sector, or the general path's reflection vector; 64 KB: two
-  // workgroups per CU
+  __shared__ int mxw[kQrWaves];
+  // X of a small sector, or the general path's reflection vector
   constexpr int kCap = kQrLds;
   __shared__ double buf[kCap];
   __shared__ double scal[6][kSmallCols];
@@ -1297,20 +1351,24 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
   const int tid = threadIdx.x;
   if (phases == kPhAll && qr_in_lds(m, n, right, C)) {
     const SmallQr<C> f{buf, buf + p * r, scal, p, r, k};
+    int mx = 0;
     for (int e = tid; e < p * r; e += kQrThreads) {
       // neighbouring threads read neighbouring elements of M
       const int i = right ? e / r : e % p, j = right ? e % r : e / p;
       const int64_t src = t.a_off + (right ? j + (int64_t)i * t.lda : i + (int64_t)j * t.lda);
-      f.re(i, j) = M[src];
-      if (C) f.im(i, j) = right ? -M[m_plane + src] : M[m_plane + src];
+      const double x = M[src], y = C ? M[m_plane + src] : 0.0;
+      mx = max(mx, max(magnitude(x), magnitude(y)));
+      f.re(i, j) = x;
+      if (C) f.im(i, j) = right ? -y : y;
     }
+    const double scale = sector_scale(group_max<kQrThreads>(mx, mxw));
     f.template factor<kQrThreads>();
     for (int e = tid; e < k * r; e += kQrThreads) {
       const int i = right ? e / r : e % k, c = right ? e % r : e / k;
       // V^dagger (k x n) = R, or U (m x k) = R^H: U[c, i] = conj(R[i, c])
       double* const o = right ? U + t.u_off + c + (int64_t)i * m : Vt + t.vt_off + i + (int64_t)c * k;
-      o[0] = f.r_re(i, c);
-      if (C) o[right ? u_plane : vt_plane] = right ? -f.r_im(i, c) : f.r_im(i, c);
+      o[0] = scale * f.r_re(i, c);
+      if (C) o[right ? u_plane : vt_plane] = scale * (right ? -f.r_im(i, c) : f.r_im(i, c));
     }
     for (int i = tid; i < k; i += kQrThreads) S[t.s_off + i] = 1.0;
     const int lane = tid & 63;
@@ -1338,17 +1396,25 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
   Mat<C> X{W + t.w_off, W + t.w_off + w_plane, p};
   Mat<C> Hv{W + t.w_off + (int64_t)p * r, W + t.w_off + (int64_t)p * r + w_plane, p};
   double* const beta = W + t.w_off + (int64_t)p * r + (int64_t)p * k;
+  double* const state = beta + k;  // the sector's scale, for the phases
+  double scale = 1.0;
   // phases: kPhLoad, kPhReflect, kPhInit (R out, Q := [I; 0]), kPhApply, kPhOut
   // (the multi-workgroup path runs the reflections and the apply in
   // house_panel/update_kernel and house_apply_kernel between them)
   if (phases & kPhLoad) {
+    int mx = 0;
     for (int64_t e = tid; e < (int64_t)p * r; e += kQrThreads) {
       const int i = (int)(e % p), j = (int)(e / p);
-      const int64_t src = right ? (j + (int64_t)i * t.lda) : (i + (int64_t)j * t.lda);
-      X.r(i, j) = M[t.a_off + src];
-      if (C) X.m(i, j) = right ? -M[t.a_off + m_plane + src] : M[t.a_off + m_plane + src];
+      const int64_t src = t.a_off + (right ? (j + (int64_t)i * t.lda) : (i + (int64_t)j * t.lda));
+      const double x = M[src], y = C ? M[m_plane + src] : 0.0;
+      mx = max(mx, max(magnitude(x), magnitude(y)));
+      X.r(i, j) = x;
+      if (C) X.m(i, j) = right ? -y : y;
     }
-    __syncthreads();
+    scale = sector_scale(group_max<kQrThreads>(mx, mxw));
+    if (tid == 0) *state = scale;
+  } else {
+    scale = *state;
   }
   if (phases & kPhReflect) house_reflect<C, kQrThreads>(X, Hv, beta, p, r, red, hv, vl);
   // R (k x r) = the upper trapezoid of X; written before X is reused for Q
@@ -1359,8 +1425,8 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
   if (phases & kPhInit) {
   for (int64_t e = tid; e < (int64_t)k * r; e += kQrThreads) {
     const int i = (int)(e % k), c = (int)(e / k);
-    const double rr = i <= c ? X.r(i, c) : 0.0;
-    const double ri = (C && i <= c) ? X.m(i, c) : 0.0;
+    const double rr = scale * (i <= c ? X.r(i, c) : 0.0);
+    const double ri = (C && i <= c) ? scale * X.m(i, c) : 0.0;
     if (!right) {  // V^dagger (k x n) = R
       Vr[i + (int64_t)c * k] = rr;
       if (C) Vi[i + (int64_t)c * k] = ri;

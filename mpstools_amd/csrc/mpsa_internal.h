@@ -137,11 +137,17 @@ hipError_t launch_colnorms(const double* A, int64_t rows, int64_t cols, int64_t 
 // ld k) at vt_off, k = min(m, n); workspace at w_off of svd_workspace(m, n)
 // elements per plane (p = max(m, n), r = min(m, n) <= kSvdMaxR: X and the
 // QR's reflection vectors, p x r each, the rotated R^H and the accumulated
-// rotations, r x r each, and r betas).  Complex data planar.
+// rotations, r x r each, r betas and a scale).  Complex data planar.  U, S and
+// V^dagger of a matrix that holds a value that is not finite are NaN.
 constexpr int kSvdMaxR = 1024;
 inline int64_t svd_workspace(int64_t m, int64_t n) {
   const int64_t p = m > n ? m : n, r = m > n ? n : m;
-  return 2 * p * r + 2 * r * r + r;
+  return 2 * p * r + 2 * r * r + r + 1;
+}
+// The QR's (LQ's when right) workspace: X, the reflection vectors, betas, a scale.
+inline int64_t qr_workspace(int64_t m, int64_t n, int right) {
+  const int64_t k = m > n ? n : m;
+  return m * n + (right ? n : m) * k + k + 1;
 }
 struct SvdTask {
   int64_t a_off, u_off, vt_off, s_off, w_off;

@@ -508,8 +508,7 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
     std::vector<double> sv((size_t)std::max<int64_t>(tot_S, 1));
     if (tot_S) hchk(hipMemcpyAsync(sv.data(), Sg.p, sizeof(double) * tot_S, hipMemcpyDeviceToHost, st), "split: S");
     hchk(hipStreamSynchronize(st), "split: sync");
-    // the batched SVD's sweeps end at once on columns of NaN, which gesvdj
-    // reports as not converged
+    // NaN: a sector that the batched SVD has no factors of
     for (auto& kv : secs) {
       const Sector& S = kv.second;
       if (dm_route(S) || !own_svd(S.m, S.n)) continue;

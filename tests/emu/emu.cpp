@@ -1118,7 +1118,7 @@ hipError_t launch_qr_batched(int cplx, int right, const SvdTask* tasks, int ntas
         ok = chk_range(U, t.u_off + q * u_plane, t.u_off + q * u_plane + (int64_t)m * k - 1, "qr U") && ok;
         ok = chk_range(Vt, t.vt_off + q * vt_plane, t.vt_off + q * vt_plane + (int64_t)k * n - 1, "qr Vt") && ok;
         ok = chk_range(W, t.w_off + q * w_plane,
-                       t.w_off + q * w_plane + (int64_t)p * r + (int64_t)p * k + k - 1, "qr W") && ok;
+                       t.w_off + q * w_plane + qr_workspace(m, n, right) - 1, "qr W") && ok;
       }
       ok = chk_range(S, t.s_off, t.s_off + k - 1, "qr S") && ok;
       if (!ok) return;
@@ -1167,9 +1167,12 @@ hipError_t launch_qr_batched(int cplx, int right, const SvdTask* tasks, int ntas
         base[off] = z.real();
         if (cplx) base[off + plane] = z.imag();
       };
+      bool finite = true;
+      for (int j = 0; j < n; ++j)
+        for (int i = 0; i < m; ++i) finite = finite && std::isfinite(std::abs(mat(i, j)));
       for (int c = 0; c < r; ++c)
         for (int i = 0; i < k; ++i) {
-          const Z rv = i <= c ? X[(size_t)i + (size_t)c * p] : Z(0.0);
+          const Z rv = !finite ? Z(NAN, NAN) : i <= c ? X[(size_t)i + (size_t)c * p] : Z(0.0);
           if (!right) put(Vt, vt_plane, t.vt_off + i + (int64_t)c * k, rv);
           else put(U, u_plane, t.u_off + c + (int64_t)i * m, std::conj(rv));
         }
@@ -1185,7 +1188,8 @@ hipError_t launch_qr_batched(int cplx, int right, const SvdTask* tasks, int ntas
   return hipSuccess;
 }
 // batched thin SVD (mpsa_factor.hip's contract): LAPACK dgesvd / zgesvd per
-// task, singular values descending, FixPhase on real data
+// task, singular values descending, FixPhase on real data; every output NaN
+// where the matrix holds a value that is not finite
 hipError_t launch_svd_batched(int cplx, const SvdTask* tasks, int ntasks, const double* M, int64_t m_plane, double* U,
                               int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W, int64_t w_plane,
                               hipStream_t st) {
@@ -1220,6 +1224,18 @@ hipError_t launch_svd_batched(int cplx, const SvdTask* tasks, int ntasks, const 
       }
       ok = chk_range(S, t.s_off, t.s_off + k - 1, "svd S") && ok;
       if (!ok) return;
+      bool finite = true;
+      for (int q = 0; q < pl; ++q)
+        for (int j = 0; j < n; ++j)
+          for (int i = 0; i < m; ++i) finite = finite && std::isfinite(M[t.a_off + q * m_plane + i + (int64_t)j * t.lda]);
+      if (!finite) {
+        for (int q = 0; q < pl; ++q) {
+          std::fill_n(U + t.u_off + q * u_plane, (size_t)m * k, NAN);
+          std::fill_n(Vt + t.vt_off + q * vt_plane, (size_t)k * n, NAN);
+        }
+        std::fill_n(S + t.s_off, (size_t)k, NAN);
+        continue;
+      }
       int mm = m, nn = n, lda = m, ldu = m, ldvt = k, lwork = -1, info = 0;
       if (!cplx) {
         std::vector<double> a((size_t)m * n), u((size_t)m * k), vt((size_t)k * n), s((size_t)k);

@@ -28,7 +28,7 @@ import scipy.sparse.linalg
 import dense
 import problems
 import pydmrg
-from mpstools_amd import models, native
+from mpstools_amd import models, native, synth
 from test_oracle import _sector_H, right_normalised_mps
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -380,6 +380,41 @@ def test_emulated_split_matches_oracle(lib, oracle, model, L, N, D, seed, dense,
     for key in left.keys():
         wgt = np.asarray(lam[key[1]]) / lmax
         assert np.max(np.abs((got["left"][key] - left[key]) * wgt[None, :]), initial=0.0) <= 1e-10, key
+
+
+def test_emulated_factorisations_refuse_nan(lib, oracle):
+    """A NaN in a two-site state's sector (its first or last entry) or in an MPS
+    is an error of the split and of the Chebyshev engine's compression, whose
+    sector SVDs answer with NaN."""
+    P = problems.build(oracle, "xxz", 8, 4, 10, 71)
+    c, itk, psi = P["c"], P["itk"], P["psi"]
+    itl, itr = native._itk(itk[c]), native._itk(itk[c + 1])
+    t = native.Table.from_blocks(psi)
+    for at in (None, 0, t.total - 1):
+        x = t.pack(psi)
+        if at is not None:
+            x[at] = np.nan
+        h = C.c_void_p()
+        rc = native.lib().mpsa_split(C.byref(t.s), DevBuf(lib, x).p, native._ptr(itl), len(itl), native._ptr(itr),
+                                     len(itr), 1, 10 ** 6, 0, 0.0, 1, C.byref(h), C.c_void_p(0))
+        assert (rc != 0) == (at is not None)
+        if rc == 0:
+            native.lib().mpsa_split_destroy(h)
+    L = 5
+    itk = [models.itokey_u1()] * L
+    mps, _ = synth.random_mps(L, itk, 2, 6, 9)
+    for bad in (False, True):
+        if bad:
+            k = sorted(mps[2].keys())[-1]
+            mps[2].b[k] = mps[2].b[k].copy()
+            mps[2].b[k][-1, -1] = np.nan
+        eng = native.Cheb([mps], models.xxz_mpo(L, 1.0, 1.0, 0.0), itk, alloc=lambda a: DevBuf(lib, a),
+                          to_host=lambda b: b.host())
+        if bad:
+            with pytest.raises(native.MpsaError, match="did not converge"):
+                eng.compress(0, 4)
+        else:
+            eng.compress(0, 4)
 
 
 def test_emulated_chebyshev_moments_match_spectral_sum(lib, oracle):

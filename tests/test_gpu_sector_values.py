@@ -1,0 +1,103 @@
+"""Sector factorisations of values at the ends of the doubles' range: entries
+that are not finite."""
+import numpy as np
+import pytest
+
+import factorcase
+from mpstools_amd import models, native, synth
+from mpstools_amd.blocks import Blocks
+
+pytestmark = pytest.mark.gpu
+
+NAN, INF = float("nan"), float("inf")
+
+
+def one_sector(M, s1=2, s2=2, l=0):
+    """A two-site state whose only sector is M (rows by s1, columns by s2)."""
+    m, n = M.shape[0] // s1, M.shape[1] // s2
+    psi = Blocks(2)
+    for a in range(s1):
+        for b in range(s2):
+            psi[(l, l, a, b)] = np.asfortranarray(M[a * m:(a + 1) * m, b * n:(b + 1) * n])
+    return psi
+
+
+def split(torch, psi, **kw):
+    t = native.Table.from_blocks(psi)
+    return native.split(t, torch.from_numpy(t.pack(psi)).cuda(), [0, 0], [0, 0], direction=1, chimax=10 ** 6, **kw)
+
+
+# one singular value (both ways), two, a sector in one workgroup's LDS, one
+# beyond it, two of several workgroups (the longest that they take)
+SHAPES = [(1, 14), (14, 1), (2, 14), (30, 40), (30, 600), (64, 80), (40, 1024)]
+
+
+@pytest.mark.parametrize("value", [NAN, INF, -INF])
+@pytest.mark.parametrize("m,n", SHAPES)
+@pytest.mark.parametrize("last", [False, True])
+def test_split_refuses_what_is_not_finite(gpu, m, n, last, value):
+    """One bad entry in the first or the last row and column of one of two
+    sectors is an error, as a sector of rocSOLVER's that does not converge is."""
+    print("[case] split", m, n, last, value, flush=True)
+    rng = np.random.default_rng(5 * m + n)
+    M = rng.standard_normal((m, n))
+    at = (m - 1, n - 1) if last else (0, 0)
+    s1, s2 = (1 if m % 2 else 2), (1 if n % 2 else 2)
+    psi = one_sector(rng.standard_normal((6, 8)), 2, 2, l=4)
+    for bad in (False, True):
+        if bad:
+            M[at] = value
+        for k, b in one_sector(M, s1, s2).b.items():
+            psi[k] = b
+        if bad:
+            with pytest.raises(native.MpsaError, match="did not converge"):
+                split(gpu, psi)
+        else:
+            assert split(gpu, psi)["chi"] == min(m, n) + 6
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("blocked", [False, True])
+def test_outputs_of_a_sector_that_is_not_finite(gpu, cplx, blocked):
+    """NaN in every output of the SVD and in R of the QR (L of the LQ), for a
+    bad entry at either end and of either plane; the sectors beside it keep
+    their factors."""
+    rng = np.random.default_rng(17)
+    draw = lambda m, n: rng.standard_normal((m, n)) + (1j * rng.standard_normal((m, n)) if cplx else 0.0)  # noqa: E731
+    shapes = [(40, 33), (33, 50)] if blocked else [(1, 9), (9, 1), (2, 2), (30, 12), (12, 31), (600, 7)]
+    for m, n in shapes:
+        for at in ((0, 0), (m - 1, n - 1)):
+            for value in (NAN, INF) + ((1j * NAN, 1j * INF) if cplx else ()):
+                bad = draw(m, n)
+                bad[at] = value
+                mats = [draw(m, n), bad, draw(n, m)]
+                for right in (None, False, True):
+                    print("[case]", m, n, at, value, right, flush=True)
+                    case = factorcase.Case(gpu, mats, right)
+                    got = case.blocked() if blocked else case.batched()
+                    for i in (0, 2):
+                        U, S, Vh = got[i]
+                        assert np.max(np.abs((U * S) @ Vh - mats[i])) <= 1e-12
+                    U, S, Vh = got[1]
+                    if right is None:
+                        assert np.all(np.isnan(U.real)) and np.all(np.isnan(S)) and np.all(np.isnan(Vh.real))
+                    else:
+                        assert np.all(np.isnan((U if right else Vh).real))
+
+
+def test_compression_refuses_what_is_not_finite(gpu):
+    """The Chebyshev engine's compression of a state with a NaN is an error."""
+    L = 6
+    itk = [models.itokey_u1xu1()] * L
+    mps, _ = synth.random_mps(L, itk, models.pack_charge(L // 2, L // 2), 8, 3)
+    for bad in (False, True):
+        if bad:
+            k = sorted(mps[2].keys())[-1]
+            mps[2].b[k] = mps[2].b[k].copy()
+            mps[2].b[k][-1, -1] = NAN
+        eng = native.Cheb([mps], models.hubbard_mpo(L, 1.0, 2.0), itk)
+        if bad:
+            with pytest.raises(native.MpsaError, match="did not converge"):
+                eng.compress(0, 6)
+        else:
+            eng.compress(0, 6)
