@@ -23,8 +23,8 @@
 // Singular vectors of exactly zero singular values (on the Z side; Q Wm is
 // orthonormal by construction) are completed to an orthonormal basis
 // (Gram-Schmidt of unit vectors, twice), as a LAPACK thin SVD returns them.
-// A sector whose matrix holds a value that is not finite has NaN in every
-// output.
+// A sector whose matrix holds a value that is not finite, or that still rotates
+// after max_sweeps sweeps, has NaN in every output.
 // Real data: FixPhase makes the first largest-|.| entry of every row of
 // V^dagger positive (the column of U flips with it).
 //
@@ -83,8 +83,8 @@ __device__ __forceinline__ int group_max(int x, int* red) {
   return x;
 }
 // What a sector's values are multiplied by at the outputs: NaN where its
-// matrix holds a value that is not finite, so that no caller takes the
-// factors for a result.
+// matrix holds a value that is not finite (or the sweeps reach their limit), so
+// that no caller takes the factors for a result.
 __device__ __forceinline__ double sector_scale(int mx) {
   return mx >= kNotFinite ? __longlong_as_double(0x7ff8000000000000ll) : 1.0;
 }
@@ -487,16 +487,17 @@ struct SmallQr {
 // One-sided Jacobi sweeps on the r <= 64 columns of A (r x r, ld r) with the
 // rotations accumulated in w, all in LDS: the pairing, rotation and stopping
 // rule of svd_jacobi_kernel's sweeps, one row per lane.  Starts and ends with
-// a barrier; flag: one LDS integer.
+// a barrier; flag: one LDS integer.  False when the last sweep still rotated.
 template <bool C, int NT>
-__device__ __forceinline__ void jacobi_small(double* ar, double* ai, double* wr, double* wi, int r, int max_sweeps,
+__device__ __forceinline__ bool jacobi_small(double* ar, double* ai, double* wr, double* wi, int r, int max_sweeps,
                                              int* flag) {
   constexpr int NW = NT / 64;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const double tol = sqrt((double)r) * DBL_EPSILON;
   const int rr = r + (r & 1);
   __syncthreads();
-  for (int sweep = 0; sweep < max_sweeps && r > 1; ++sweep) {
+  if (r <= 1) return true;
+  for (int sweep = 0; sweep < max_sweeps; ++sweep) {
     if (threadIdx.x == 0) *flag = 0;
     __syncthreads();
     for (int round = 0; round < rr - 1; ++round) {
@@ -549,8 +550,9 @@ __device__ __forceinline__ void jacobi_small(double* ar, double* ai, double* wr,
     }
     const int any = *flag;
     __syncthreads();
-    if (!any) break;
+    if (!any) return true;
   }
+  return false;
 }
 
 static_assert(kSmallRows == 512 && kSmallCols == 64 && kQrLds + 6 * kSmallCols <= 8192, "qr_in_lds states these limits");
@@ -628,7 +630,8 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
         lw[r * r + e] = 0.0;
       }
     }
-    jacobi_small<C, kThreads>(la, la + r * r, lw, lw + r * r, r, max_sweeps, &rotated);
+    if (!jacobi_small<C, kThreads>(la, la + r * r, lw, lw + r * r, r, max_sweeps, &rotated))
+      scale = sector_scale(kNotFinite);
     for (int c = wave; c < r; c += kWaves) {
       double yr[kSmallRpl], yi[kSmallRpl];
 #pragma unroll
@@ -688,7 +691,8 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
   if (phases & kPhSweep) {
   const double tol = sqrt((double)r) * DBL_EPSILON;
   const int rr = r + (r & 1);
-  for (int sweep = 0; sweep < max_sweeps && r > 1; ++sweep) {
+  bool ended = r <= 1;
+  for (int sweep = 0; sweep < max_sweeps && !ended; ++sweep) {
     if (tid == 0) rotated = 0;
     __syncthreads();
     for (int round = 0; round < rr - 1; ++round) {
@@ -753,10 +757,10 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
       }
       __syncthreads();
     }
-    const int any = rotated;
+    ended = !rotated;
     __syncthreads();
-    if (!any) break;
   }
+  if (!ended) scale = sector_scale(kNotFinite);
   }
   // X = Q [Wm; 0]: the accumulated rotations back through the reflections
   if (phases & kPhBackInit) {
@@ -1771,10 +1775,10 @@ hipError_t launch_svd_phase(int cplx, int phases, const SvdTask* tasks, int ntas
   if (ntasks <= 0) return hipSuccess;
   if (cplx)
     svd_jacobi_kernel<true><<<ntasks, kThreads, 0, st>>>(tasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane,
-                                                          60, phases);
+                                                          kSvdSweeps, phases);
   else
     svd_jacobi_kernel<false><<<ntasks, kThreads, 0, st>>>(tasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W,
-                                                           w_plane, 60, phases);
+                                                           w_plane, kSvdSweeps, phases);
   return hipGetLastError();
 }
 
@@ -1866,14 +1870,14 @@ int svd_block_rounds(int m, int n) {
 
 hipError_t launch_svd_batched(int cplx, const SvdTask* tasks, int ntasks, const double* M, int64_t m_plane,
                               double* U, int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W,
-                              int64_t w_plane, hipStream_t st) {
+                              int64_t w_plane, hipStream_t st, int max_sweeps) {
   if (ntasks <= 0) return hipSuccess;
   if (cplx)
     svd_jacobi_kernel<true><<<ntasks, kThreads, 0, st>>>(tasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane,
-                                                          60, kPhAll);
+                                                          max_sweeps, kPhAll);
   else
     svd_jacobi_kernel<false><<<ntasks, kThreads, 0, st>>>(tasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W,
-                                                           w_plane, 60, kPhAll);
+                                                           w_plane, max_sweeps, kPhAll);
   return hipGetLastError();
 }
 

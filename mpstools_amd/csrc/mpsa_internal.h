@@ -138,8 +138,10 @@ hipError_t launch_colnorms(const double* A, int64_t rows, int64_t cols, int64_t 
 // elements per plane (p = max(m, n), r = min(m, n) <= kSvdMaxR: X and the
 // QR's reflection vectors, p x r each, the rotated R^H and the accumulated
 // rotations, r x r each, r betas and a scale).  Complex data planar.  U, S and
-// V^dagger of a matrix that holds a value that is not finite are NaN.
+// V^dagger are NaN where the matrix holds a value that is not finite or the
+// last of max_sweeps sweeps still rotated.
 constexpr int kSvdMaxR = 1024;
+constexpr int kSvdSweeps = 60;  // several times what converging sectors need
 inline int64_t svd_workspace(int64_t m, int64_t n) {
   const int64_t p = m > n ? m : n, r = m > n ? n : m;
   return 2 * p * r + 2 * r * r + r + 1;
@@ -155,7 +157,7 @@ struct SvdTask {
 };
 hipError_t launch_svd_batched(int cplx, const SvdTask* tasks, int ntasks, const double* M, int64_t m_plane,
                               double* U, int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W,
-                              int64_t w_plane, hipStream_t st);
+                              int64_t w_plane, hipStream_t st, int max_sweeps = kSvdSweeps);
 // Sectors that launch_qr_batched factorises in one workgroup's LDS: at most 512
 // rows and 64 columns of X (M, or M^H when right), kQrLds doubles.
 constexpr int kQrLds = 7808;

@@ -29,7 +29,7 @@ inline int house_table(const std::vector<SvdTask>& ts, int layout, std::vector<i
 //   void check(hipError_t, const char*)     throws on an error
 //   void wait()                             drains the stream
 // flags: big.size() doubles of device memory, zero.  False when a sector still
-// rotates after 60 sweeps.
+// rotates after kSvdSweeps sweeps.
 template <class Dev>
 bool svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const double* M, int64_t m_plane, double* U,
                      int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W, int64_t w_plane,
@@ -49,7 +49,7 @@ bool svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const
   // sector leaves it as it is, so later sweeps would not rotate it either
   std::vector<SvdTask> act = big;
   std::vector<double> hf((size_t)nb);
-  for (int sweep = 0; sweep < 60 && !act.empty(); ++sweep) {
+  for (int sweep = 0; sweep < kSvdSweeps && !act.empty(); ++sweep) {
     const int na = (int)act.size();
     std::vector<int> base((size_t)na + 1, 0);
     int rounds = 0, rmax = 1;

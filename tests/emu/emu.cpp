@@ -47,6 +47,7 @@ struct Alloc {
 std::map<uintptr_t, Alloc> g_alloc;
 long g_serial = 0, g_viol = 0, g_launch = 0;
 std::string g_ctx = "-";
+bool g_rotating = false;  // every block round rotates: a sector SVD that does not converge
 std::vector<std::string> g_msgs;
 
 void report(const std::string& m) {
@@ -130,6 +131,7 @@ extern "C" {
 long emu_violations() { return g_viol; }
 const char* emu_message(int i) { return i < (int)g_msgs.size() ? g_msgs[(size_t)i].c_str() : nullptr; }
 long emu_launches() { return g_launch; }
+void emu_set_rotating(int on) { g_rotating = on != 0; }
 long emu_live_bytes() {
   long b = 0;
   for (auto& kv : g_alloc)
@@ -1192,7 +1194,7 @@ hipError_t launch_qr_batched(int cplx, int right, const SvdTask* tasks, int ntas
 // where the matrix holds a value that is not finite
 hipError_t launch_svd_batched(int cplx, const SvdTask* tasks, int ntasks, const double* M, int64_t m_plane, double* U,
                               int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W, int64_t w_plane,
-                              hipStream_t st) {
+                              hipStream_t st, int) {
   if (ntasks <= 0) return hipSuccess;
   submit(st, "svd batched", [=]() {
     if (!chk_range(tasks, 0, ntasks - 1, "svd tasks")) return;
@@ -1313,7 +1315,7 @@ hipError_t launch_svd_phase(int cplx, int phases, const SvdTask* tasks, int ntas
     chk_phase_tasks(st, tasks, ntasks, kSvdBlockMaxR);
     return hipSuccess;
   }
-  return launch_svd_batched(cplx, tasks, ntasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane, st);
+  return launch_svd_batched(cplx, tasks, ntasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane, st, kSvdSweeps);
 }
 hipError_t launch_qr_phase(int cplx, int right, int phases, const SvdTask* tasks, int ntasks, const double* M,
                            int64_t m_plane, double* U, int64_t u_plane, double* Vt, int64_t vt_plane, double* S,
@@ -1364,6 +1366,8 @@ hipError_t launch_svd_block_round(int, const SvdTask* tasks, int ntasks, const i
         !chk_range(rotated, 0, ntasks - 1, "svd rotated"))
       return;
     if (pair_base[0] != 0 || pair_base[ntasks] != npairs || round < -1) report("svd block round: bad pair table");
+    if (g_rotating)
+      for (int i = 0; i < ntasks; ++i) rotated[i] = 1.0;
   });
   return hipSuccess;
 }

@@ -76,12 +76,12 @@ class Case:
     def _st(self):
         return native._stream()
 
-    def batched(self):
+    def batched(self, max_sweeps=60):
         """All sectors in one launch, one workgroup each."""
         c, n, t = int(self.cplx), len(self.mats), C.c_void_p(self.dt.data_ptr())
         if self.right is None:
-            self._call(_fn("launch_svd_batched", "iPKNS_7SvdTaskEi" + _ARRAYS + "P12ihipStream_t"), c, t, n,
-                       *self._arrays(), self._st())
+            self._call(_fn("launch_svd_batched", "iPKNS_7SvdTaskEi" + _ARRAYS + "P12ihipStream_ti"), c, t, n,
+                       *self._arrays(), self._st(), max_sweeps)
         else:
             self._call(_fn("launch_qr_batched", "iiPKNS_7SvdTaskEi" + _ARRAYS + "P12ihipStream_t"), c,
                        int(self.right), t, n, *self._arrays(), self._st())

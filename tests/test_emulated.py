@@ -29,6 +29,7 @@ import dense
 import problems
 import pydmrg
 from mpstools_amd import models, native, synth
+from mpstools_amd.blocks import Blocks
 from test_oracle import _sector_H, right_normalised_mps
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -415,6 +416,40 @@ def test_emulated_factorisations_refuse_nan(lib, oracle):
                 eng.compress(0, 4)
         else:
             eng.compress(0, 4)
+
+
+def test_emulated_sector_svds_that_do_not_converge(lib, oracle):
+    """Block rounds that never stop rotating end at the sweep limit with the
+    error of the split and of the Chebyshev engine."""
+    rng = np.random.default_rng(5)
+    psi = Blocks(2)
+    for s1 in range(2):
+        for s2 in range(2):
+            psi[(0, 0, s1, s2)] = np.asfortranarray(rng.standard_normal((17, 18)))  # 34 x 36
+    itk = native._itk([0, 0])
+    t = native.Table.from_blocks(psi)
+    L = 5
+    mps, itks = right_normalised_mps(L, 2, 6, 9)
+    eng = native.Cheb([mps], models.xxz_mpo(L, 1.0, 1.0, 0.0), itks, alloc=lambda a: DevBuf(lib, a),
+                      to_host=lambda b: b.host())
+    eng.set_big_sector(1000)
+    eng.set_block_jacobi(2)
+    for on in (1, 0):
+        lib.emu_set_rotating(on)
+        try:
+            h = C.c_void_p()
+            rc = native.lib().mpsa_split(C.byref(t.s), DevBuf(lib, t.pack(psi)).p, native._ptr(itk), 2,
+                                         native._ptr(itk), 2, 1, 10 ** 6, 0, 0.0, 1, C.byref(h), C.c_void_p(0))
+            assert (rc != 0) == bool(on)
+            if rc == 0:
+                native.lib().mpsa_split_destroy(h)
+            if on:
+                with pytest.raises(native.MpsaError, match="did not converge"):
+                    eng.compress(0, 4)
+            else:
+                eng.compress(0, 4)
+        finally:
+            lib.emu_set_rotating(0)
 
 
 def test_emulated_chebyshev_moments_match_spectral_sum(lib, oracle):

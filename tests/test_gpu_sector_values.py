@@ -1,5 +1,5 @@
-"""Sector factorisations of values at the ends of the doubles' range: entries
-that are not finite."""
+"""Sector factorisations that have no result: entries that are not finite,
+sweeps that reach their limit."""
 import numpy as np
 import pytest
 
@@ -83,6 +83,24 @@ def test_outputs_of_a_sector_that_is_not_finite(gpu, cplx, blocked):
                         assert np.all(np.isnan(U.real)) and np.all(np.isnan(S)) and np.all(np.isnan(Vh.real))
                     else:
                         assert np.all(np.isnan((U if right else Vh).real))
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+def test_sweeps_at_their_limit(gpu, cplx):
+    """A sector that still rotates in its last sweep answers with NaN (in LDS and
+    beyond it); one sweep is enough where nothing rotates."""
+    rng = np.random.default_rng(23)
+    shapes = [(2, 2), (12, 30), (30, 12), (600, 7), (40, 70)]
+    mats = [rng.standard_normal(s) + (1j * rng.standard_normal(s) if cplx else 0.0) for s in shapes]
+    mats += [np.eye(9, 4), rng.standard_normal((1, 5)), rng.standard_normal((5, 1))]
+    print("[case] sweeps", cplx, flush=True)
+    for sweeps in (1, 60):
+        got = factorcase.Case(gpu, mats).batched(sweeps)
+        for i, (U, S, Vh) in enumerate(got):
+            if sweeps == 1 and i < len(shapes):
+                assert np.all(np.isnan(S)) and np.all(np.isnan(U.real)) and np.all(np.isnan(Vh.real))
+            else:
+                assert np.max(np.abs((U * S) @ Vh - mats[i])) <= 1e-13
 
 
 def test_compression_refuses_what_is_not_finite(gpu):
