@@ -82,11 +82,33 @@ __device__ __forceinline__ int group_max(int x, int* red) {
   for (int w = 0; w < NT / 64; ++w) x = max(x, red[w]);
   return x;
 }
-// What a sector's values are multiplied by at the outputs: NaN where its
-// matrix holds a value that is not finite (or the sweeps reach their limit), so
-// that no caller takes the factors for a result.
+// What a sector's values are multiplied by at the outputs (its loads by 1 /
+// scale).  A power of two near its largest entry where that lies outside
+// 2^-300 .. 2^300, so that the squares of its entries stay in the range of
+// doubles; else 1.  NaN where its matrix holds a value that is not finite (or
+// the sweeps reach their limit), so that no caller takes the factors for a
+// result.
 __device__ __forceinline__ double sector_scale(int mx) {
-  return mx >= kNotFinite ? __longlong_as_double(0x7ff8000000000000ll) : 1.0;
+  if (mx >= kNotFinite) return __longlong_as_double(0x7ff8000000000000ll);
+  const int e = mx >> 20;  // exponent + 1023
+  return e > 723 && e < 1323 ? 1.0 : __hiloint2double(min(max(e, 1), 2045) << 20, 0);
+}
+// Columns of squared norm below this count as zero: with the largest entry at
+// 2^-300 or above they are less than 2^-140 of it, and their reciprocal
+// squares and products would leave the range of doubles.
+constexpr double kTinySq = 0x1p-880;
+// A column's head of |x|^2 below this has phase 1 in its reflection: its
+// square has lost bits, and it is less than 2^-60 of a column that is not zero.
+constexpr double kPhaseSq = 0x1p-1000;
+// |x| and the unit phase of a column's head, for its reflection
+template <bool C>
+__device__ __forceinline__ double head_phase(double xr, double xi, double& er, double& ei) {
+  const double s = xr * xr + xi * xi;
+  const double a = C ? sqrt(s) : fabs(xr);
+  const bool ok = C ? s >= kPhaseSq : a > 0.0;
+  er = ok ? xr / a : 1.0;
+  ei = C && ok ? xi / a : 0.0;
+  return a;
 }
 
 // Column j of a p-row matrix with leading dimension ld, planar complex.
@@ -129,11 +151,11 @@ __device__ __forceinline__ void rotate_cols(const Mat<C>& X, int p, int i, int j
 // with d = b - a, h = 2 |g| is the smaller root of the rotation's quadratic; two
 // square roots and one division, where the quotient form takes three of each
 // in a chain that a whole round waits for.  Columns whose products could leave
-// the range of doubles take that form.
+// the range of doubles take that form; those below kTinySq are not rotated.
 template <bool C>
 __device__ __forceinline__ bool jacobi_rotation(double a, double b, double gr, double gi, double tol, double& c,
                                                 double& sn, double& er, double& ei) {
-  if (a == 0.0 || b == 0.0) return false;
+  if (!(a >= kTinySq && b >= kTinySq)) return false;
   if (a > 1e-120 && b > 1e-120 && a < 1e120 && b < 1e120) {
     const double g2 = gr * gr + (C ? gi * gi : 0.0);
     if (!(g2 > tol * tol * (a * b))) return false;
@@ -159,7 +181,8 @@ __device__ __forceinline__ bool jacobi_rotation(double a, double b, double gr, d
   er = gr / g;
   ei = C ? gi / g : 0.0;
   const double zeta = (b - a) / (2.0 * g);
-  const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
+  const double t = fabs(zeta) > 1e100 ? 0.5 / zeta  // zeta^2 may overflow
+                                      : (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
   c = 1.0 / sqrt(1.0 + t * t);
   sn = c * t;
   return true;
@@ -239,7 +262,7 @@ __device__ __forceinline__ void reflect_col_global(const Mat<C>& Y, int c, int f
 // Householder reflections of X (p x r, planar, ld p) in place, one per
 // column j < k = min(p, r): H_j = I - beta_j v_j v_j^H with v_j = x - alpha e_j,
 // alpha = -e^{i arg x_j} |x| (x = rows j.. of column j), beta_j = 2 / |v_j|^2
-// (0 for a zero column: H_j = I).  Column j becomes (alpha, 0, ...), the
+// (0 for a zero column, below kTinySq: H_j = I, alpha = 0).  Column j becomes (alpha, 0, ...), the
 // columns after it are reflected (one wave per column, the column in
 // registers and v_j in LDS when p - j <= kVecRows); v_j goes to rows j.. of
 // column j of Hv, beta_j to beta[j].  NT threads; red holds NT / 64 doubles,
@@ -267,10 +290,11 @@ __device__ void house_reflect(const Mat<C>& X, const Mat<C>& Hv, double* beta, i
       double nn = 0.0;
       for (int w = 0; w < NW; ++w) nn += red[w];
       const double x0r = X.r(j, j), x0i = C ? X.m(j, j) : 0.0;
-      const double a0 = sqrt(x0r * x0r + x0i * x0i), nrm = sqrt(nn);
+      const double nrm = sqrt(nn);
       double ar = 0.0, ai = 0.0, b = 0.0;
-      if (nn > 0.0) {
-        const double er = a0 > 0.0 ? x0r / a0 : 1.0, ei = a0 > 0.0 ? x0i / a0 : 0.0;
+      if (nn >= kTinySq) {
+        double er, ei;
+        const double a0 = head_phase<C>(x0r, x0i, er, ei);
         ar = -er * nrm;
         ai = -ei * nrm;
         const double v0r = x0r - ar, v0i = x0i - ai;
@@ -382,10 +406,11 @@ struct SmallQr {
     for (int j = 0; j < k; ++j) {
       const double nn = s[5][j & 1];
       const double x0r = re(j, j), x0i = C ? im(j, j) : 0.0;
-      const double a0 = C ? sqrt(x0r * x0r + x0i * x0i) : fabs(x0r), nrm = sqrt(nn);
+      const double nrm = sqrt(nn);
       double ar = 0.0, ai = 0.0, b = 0.0;
-      if (nn > 0.0) {
-        const double er = a0 > 0.0 ? x0r / a0 : 1.0, ei = a0 > 0.0 ? x0i / a0 : 0.0;
+      if (nn >= kTinySq) {
+        double er, ei;
+        const double a0 = head_phase<C>(x0r, x0i, er, ei);
         ar = -er * nrm;
         ai = -ei * nrm;
         const double v0r = x0r - ar, v0i = x0i - ai;
@@ -620,6 +645,14 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
       if (C) f.im(i, j) = wide ? -y : y;
     }
     scale = sector_scale(group_max<kThreads>(mx, mxw));
+    if (scale != 1.0) {  // uniform
+      for (int e = tid; e < p * r; e += kThreads) {
+        const int i = wide ? e / r : e % p, j = wide ? e % r : e / p;
+        f.re(i, j) /= scale;
+        if (C) f.im(i, j) /= scale;
+      }
+      __syncthreads();
+    }
     f.template factor<kThreads>();
     for (int e = tid; e < r * r; e += kThreads) {  // A = R^H, Wm = I
       const int i = e % r, j = e / r;
@@ -672,6 +705,13 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
       if (C) X.m(i, j) = wide ? -y : y;
     }
     scale = sector_scale(group_max<kThreads>(mx, mxw));
+    if (scale != 1.0) {  // uniform
+      for (int64_t e = tid; e < (int64_t)p * r; e += kThreads) {
+        X.re[e] /= scale;
+        if (C) X.im[e] /= scale;
+      }
+      __syncthreads();
+    }
     if (tid == 0) *state = scale;
   } else if (!small) {
     scale = *state;
@@ -785,7 +825,7 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
       }
     }
     a = wave_sum(a);
-    a = sqrt(a);
+    a = a < kTinySq ? 0.0 : sqrt(a);
     if (lane == 0) sig[j] = a;
     if (!(a <= DBL_MAX)) scale = a;
   }
@@ -807,7 +847,7 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
     const double sj = sig[j];
     for (int i = 0; i < r; ++i) rk += (sig[i] > sj || (sig[i] == sj && i < j)) ? 1 : 0;
     rank[j] = rk;
-    S[t.s_off + rk] = sj;
+    S[t.s_off + rk] = sj * scale;
   }
   __syncthreads();
   // U (m x k, ld m) and V^dagger (k x n, ld k): the p side from Q Wm, the r
@@ -1366,6 +1406,14 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
       if (C) f.im(i, j) = right ? -y : y;
     }
     const double scale = sector_scale(group_max<kQrThreads>(mx, mxw));
+    if (scale != 1.0) {  // uniform
+      for (int e = tid; e < p * r; e += kQrThreads) {
+        const int i = right ? e / r : e % p, j = right ? e % r : e / p;
+        f.re(i, j) /= scale;
+        if (C) f.im(i, j) /= scale;
+      }
+      __syncthreads();
+    }
     f.template factor<kQrThreads>();
     for (int e = tid; e < k * r; e += kQrThreads) {
       const int i = right ? e / r : e % k, c = right ? e % r : e / k;
@@ -1416,6 +1464,13 @@ __global__ __launch_bounds__(kQrThreads) void qr_householder_kernel(const SvdTas
       if (C) X.m(i, j) = right ? -y : y;
     }
     scale = sector_scale(group_max<kQrThreads>(mx, mxw));
+    if (scale != 1.0) {  // uniform
+      for (int64_t e = tid; e < (int64_t)p * r; e += kQrThreads) {
+        X.re[e] /= scale;
+        if (C) X.im[e] /= scale;
+      }
+      __syncthreads();
+    }
     if (tid == 0) *state = scale;
   } else {
     scale = *state;
@@ -1614,10 +1669,11 @@ __device__ __forceinline__ void panel_regs(const HView<C>& v, int j0, int j1, do
       }
       nn = wave_sum(nn);
       const double x0r = __shfl(xr[0], h, 64), x0i = C ? __shfl(xi[0], h, 64) : 0.0;
-      const double a0 = C ? sqrt(x0r * x0r + x0i * x0i) : fabs(x0r), nrm = sqrt(nn);
+      const double nrm = sqrt(nn);
       double ar = 0.0, ai = 0.0, b = 0.0;
-      if (nn > 0.0) {
-        const double er = a0 > 0.0 ? x0r / a0 : 1.0, ei = C && a0 > 0.0 ? x0i / a0 : 0.0;
+      if (nn >= kTinySq) {
+        double er, ei;
+        const double a0 = head_phase<C>(x0r, x0i, er, ei);
         ar = -er * nrm;
         ai = -ei * nrm;
         b = 1.0 / (nn + a0 * nrm);  // 2 / |v|^2, v = x + e |x| e_0

@@ -1,5 +1,5 @@
-"""Sector factorisations that have no result: entries that are not finite,
-sweeps that reach their limit."""
+"""Sector factorisations at the ends of the doubles' range: entries that are not
+finite, sweeps that reach their limit, entries whose squares leave the range."""
 import numpy as np
 import pytest
 
@@ -101,6 +101,85 @@ def test_sweeps_at_their_limit(gpu, cplx):
                 assert np.all(np.isnan(S)) and np.all(np.isnan(U.real)) and np.all(np.isnan(Vh.real))
             else:
                 assert np.max(np.abs((U * S) @ Vh - mats[i])) <= 1e-13
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("exp", [-310, -300, -160, -156, -155, -91, 91, 154, 160, 300])
+def test_extreme_entries(gpu, cplx, exp):
+    """Sectors of entries near 10^exp beside one of entries near 1: factors and
+    singular values of the matrix scaled to 1 within n eps (1e-13 at these
+    sizes); denormals (10^-310) and what is computed from them keep 43 bits."""
+    rng = np.random.default_rng(31)
+    draw = lambda m, n: rng.standard_normal((m, n)) + (1j * rng.standard_normal((m, n)) if cplx else 0.0)  # noqa: E731
+    for blocked, shapes in ((False, [(1, 6), (6, 1), (20, 9), (9, 31), (600, 7)]), (True, [(40, 33), (33, 200)])):
+        mats = [draw(*s) for s in shapes for _ in range(2)]
+        e = int(np.floor(exp / np.log10(2.0)))  # a power of two, in two factors: 2^-e may be beyond DBL_MAX
+        up = lambda a, f: a * 2.0 ** (f * (e // 2)) * 2.0 ** (f * (e - e // 2))  # noqa: E731
+        given = [up(a, 1) if i % 2 else a for i, a in enumerate(mats)]
+        for right in (None, False, True):
+            print("[case] extreme", exp, cplx, blocked, right, flush=True)
+            case = factorcase.Case(gpu, given, right)
+            got = case.blocked() if blocked else case.batched()
+            for i, (U, S, Vh) in enumerate(got):
+                down = lambda a: up(a, -1) if i % 2 else a  # noqa: E731
+                tol = 1e-12 if exp == -310 and i % 2 else 1e-13
+                if right is None:
+                    assert np.max(np.abs(down(S) - np.linalg.svd(mats[i], compute_uv=False))) <= tol * 10
+                    A = (U * down(S)) @ Vh
+                    isos = (U, Vh.conj().T)
+                else:
+                    assert np.all(S == 1.0)
+                    A = down(U) @ Vh if right else U @ down(Vh)
+                    isos = (Vh.conj().T if right else U,)
+                assert np.max(np.abs(A - mats[i])) <= tol * 30
+                for Q in isos:
+                    assert np.max(np.abs(Q.conj().T @ Q - np.eye(Q.shape[1]))) <= 1e-13
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+def test_columns_far_below_the_rest(gpu, cplx):
+    """Columns and rows down to 10^-300 of the others, in order and not: the
+    large singular values as without them, the matrix within n eps of its
+    largest entry, orthonormal vectors."""
+    rng = np.random.default_rng(37)
+    for blocked, (m, n) in ((False, (20, 9)), (False, (9, 20)), (False, (600, 6))):
+        A = rng.standard_normal((m, n)) + (1j * rng.standard_normal((m, n)) if cplx else 0.0)
+        k = min(m, n)
+        mats = []
+        for low in (-120, -157, -165, -300):
+            d = np.ones(n)
+            d[rng.permutation(n)[:k // 2]] = 10.0 ** low
+            mats.append(A * d)
+            mats.append(A * 10.0 ** np.linspace(0, low, n))
+            mats.append(A * 10.0 ** np.linspace(low, 0, m)[:, None])
+        for right in (None, False, True):
+            print("[case] graded", m, n, cplx, blocked, right, flush=True)
+            case = factorcase.Case(gpu, mats, right)
+            got = case.blocked() if blocked else case.batched()
+            for a, (U, S, Vh) in zip(mats, got):
+                top = np.max(np.abs(a))
+                assert np.max(np.abs((U * S) @ Vh - a)) <= 1e-13 * 30 * top
+                V = Vh.conj().T
+                for Q in (U[:, S > 0], V[:, S > 0]) if right is None else ((V,) if right else (U,)):
+                    assert np.max(np.abs(Q.conj().T @ Q - np.eye(Q.shape[1]))) <= 1e-13
+                if right is None:
+                    ref = np.linalg.svd(a, compute_uv=False)
+                    assert np.max(np.abs(S - ref)) <= 1e-13 * ref[0]
+
+
+def test_split_with_a_negligible_sector(gpu):
+    """A sector of entries near 10^-156 beside an ordinary one is no error: the
+    ordinary one is split as without it."""
+    rng = np.random.default_rng(41)
+    M, T = rng.standard_normal((30, 40)), rng.standard_normal((30, 40))
+    M /= np.linalg.norm(M)
+    for scale in (1e-156, 1e-310):
+        psi = one_sector(M)
+        for k, b in one_sector(T * scale, l=7).b.items():
+            psi[k] = b
+        out = split(gpu, psi)
+        assert out["chi"] == 30
+        assert np.max(np.abs(np.asarray(out["lam"][0]) - np.linalg.svd(M, compute_uv=False))) <= 1e-14
 
 
 def test_compression_refuses_what_is_not_finite(gpu):
