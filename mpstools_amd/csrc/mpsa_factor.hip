@@ -800,7 +800,10 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
     ended = !rotated;
     __syncthreads();
   }
-  if (!ended) scale = sector_scale(kNotFinite);
+  if (!ended) {
+    scale = sector_scale(kNotFinite);
+    if (tid == 0) *state = scale;
+  }
   }
   // X = Q [Wm; 0]: the accumulated rotations back through the reflections
   if (phases & kPhBackInit) {

@@ -23,15 +23,19 @@ inline int house_table(const std::vector<SvdTask>& ts, int layout, std::vector<i
 // The SVD of large sectors in phases: the load, the reflections in panels over
 // several workgroups per sector, the init, sweeps of block-tournament rounds
 // until a sweep rotates nothing (one host wait per sweep), the back-transform
-// over several workgroups, the outputs.  Dev gives
+// over several workgroups, the outputs (NaN where a sector does not converge).
+// The blocks' order of pairs converges slowly where columns are many orders of
+// magnitude apart (33 columns, half of them at 1e-60 of the others: 51 sweeps
+// against 18 in the order of the one-workgroup kernel, at 1e-90 more than 60
+// against 21), so that kernel finishes what still rotates after kSvdSweeps.
+// Dev gives
 //   const void* put(const std::vector<T>&)  a device copy ordered on the stream,
 //                                           valid until the next wait after its use
 //   void check(hipError_t, const char*)     throws on an error
 //   void wait()                             drains the stream
-// flags: big.size() doubles of device memory, zero.  False when a sector still
-// rotates after kSvdSweeps sweeps.
+// flags: big.size() doubles of device memory, zero.
 template <class Dev>
-bool svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const double* M, int64_t m_plane, double* U,
+void svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const double* M, int64_t m_plane, double* U,
                      int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W, int64_t w_plane,
                      double* flags, hipStream_t st) {
   const int nb = (int)big.size();
@@ -73,10 +77,13 @@ bool svd_blocked_run(Dev& dev, bool cplx, const std::vector<SvdTask>& big, const
     act.swap(next);
     if (!act.empty()) dev.check(launch_fill(flags, na, 0.0, st), "sector SVD flags");
   }
+  if (!act.empty())
+    dev.check(launch_svd_phase(cplx, kPhSweep, (const SvdTask*)dev.put(act), (int)act.size(), M, m_plane, U, u_plane,
+                               Vt, vt_plane, S, W, w_plane, st),
+              "sector SVD sweeps");
   phase(kPhBackInit, "sector SVD back-transform");
   dev.check(launch_house_apply(cplx, 0, t, nb, dh, hbase.back(), W, w_plane, st), "sector SVD back-transform");
   phase(kPhOut, "sector SVD outputs");
-  return act.empty();
 }
 
 }  // namespace mpsa

@@ -47,7 +47,9 @@ struct Alloc {
 std::map<uintptr_t, Alloc> g_alloc;
 long g_serial = 0, g_viol = 0, g_launch = 0;
 std::string g_ctx = "-";
-bool g_rotating = false;  // every block round rotates: a sector SVD that does not converge
+// every block round rotates: a sector SVD that does not converge (the
+// one-workgroup sweeps after them answer with NaN)
+bool g_rotating = false, g_swept = false;
 std::vector<std::string> g_msgs;
 
 void report(const std::string& m) {
@@ -1311,11 +1313,19 @@ hipError_t launch_svd_phase(int cplx, int phases, const SvdTask* tasks, int ntas
                             double* U, int64_t u_plane, double* Vt, int64_t vt_plane, double* S, double* W,
                             int64_t w_plane, hipStream_t st) {
   if (ntasks <= 0) return hipSuccess;
+  if (phases & kPhLoad) g_swept = false;
+  if (phases & kPhSweep) g_swept = true;
   if (!(phases & kPhOut)) {
     chk_phase_tasks(st, tasks, ntasks, kSvdBlockMaxR);
     return hipSuccess;
   }
-  return launch_svd_batched(cplx, tasks, ntasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane, st, kSvdSweeps);
+  launch_svd_batched(cplx, tasks, ntasks, M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane, st, kSvdSweeps);
+  if (g_rotating)
+    submit(st, "svd not converged", [=]() {
+      if (!g_swept) report("svd: sectors still rotating and not swept");
+      for (int i = 0; i < ntasks; ++i) std::fill_n(S + tasks[i].s_off, (size_t)std::min(tasks[i].m, tasks[i].n), NAN);
+    });
+  return hipSuccess;
 }
 hipError_t launch_qr_phase(int cplx, int right, int phases, const SvdTask* tasks, int ntasks, const double* M,
                            int64_t m_plane, double* U, int64_t u_plane, double* Vt, int64_t vt_plane, double* S,

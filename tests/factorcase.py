@@ -10,7 +10,7 @@ from mpstools_amd import native
 TASK = np.dtype([("a_off", np.int64), ("u_off", np.int64), ("vt_off", np.int64), ("s_off", np.int64),
                  ("w_off", np.int64), ("m", np.int32), ("n", np.int32), ("lda", np.int32), ("pad", np.int32)])
 _ARRAYS = "PKdlPdlS5_lS5_S5_l"  # M, m_plane, U, u_plane, Vt, vt_plane, S, W, w_plane
-LOAD, INIT, BACK, OUT = 1, 4, 16, 64  # the kPh* bits of mpsa_internal.h
+LOAD, INIT, SWEEP, BACK, OUT = 1, 4, 8, 16, 64  # the kPh* bits of mpsa_internal.h
 # the one-workgroup kernels' LDS, in doubles, as mpsa_factor.hip holds it
 SVD_LDS, QR_LDS = 12288, 7808
 
@@ -125,6 +125,8 @@ class Case:
                 self.rotating = bool((flags != 0).any().item())
                 if not self.rotating:
                     break
+            if self.rotating or max_sweeps == 0:
+                phase(SWEEP)
             phase(BACK)
         self._call(_fn("launch_house_apply", "iiPKNS_7SvdTaskEiPKiiPdlP12ihipStream_t"), c, layout, t, n, pb,
                    int(base[-1]), W, aw, self._st())

@@ -142,7 +142,7 @@ def test_columns_far_below_the_rest(gpu, cplx):
     large singular values as without them, the matrix within n eps of its
     largest entry, orthonormal vectors."""
     rng = np.random.default_rng(37)
-    for blocked, (m, n) in ((False, (20, 9)), (False, (9, 20)), (False, (600, 6))):
+    for blocked, (m, n) in ((False, (20, 9)), (False, (9, 20)), (False, (600, 6)), (True, (50, 33))):
         A = rng.standard_normal((m, n)) + (1j * rng.standard_normal((m, n)) if cplx else 0.0)
         k = min(m, n)
         mats = []
@@ -165,6 +165,35 @@ def test_columns_far_below_the_rest(gpu, cplx):
                 if right is None:
                     ref = np.linalg.svd(a, compute_uv=False)
                     assert np.max(np.abs(S - ref)) <= 1e-13 * ref[0]
+
+
+@pytest.mark.parametrize("m,n", [(34, 60), (80, 66), (300, 40)])
+def test_blocked_sweeps_finished_by_one_workgroup(gpu, m, n):
+    """Sectors that still rotate after the block rounds' sweeps (none, one, three
+    here) are finished in the one-workgroup kernel's order."""
+    rng = np.random.default_rng(43)
+    mats = [rng.standard_normal((m, n)), rng.standard_normal((n, m))]
+    for sweeps in (0, 1, 3):
+        print("[case] finished", m, n, sweeps, flush=True)
+        for a, (U, S, Vh) in zip(mats, factorcase.Case(gpu, mats).blocked(sweeps)):
+            ref = np.linalg.svd(a, compute_uv=False)
+            assert np.max(np.abs(S - ref)) <= 1e-13 * ref[0]
+            assert np.max(np.abs((U * S) @ Vh - a)) <= 1e-12
+            for Q in (U, Vh.T):
+                assert np.max(np.abs(Q.T @ Q - np.eye(Q.shape[1]))) <= 1e-13
+
+
+@pytest.mark.parametrize("low", [-60, -90, -120])
+def test_split_of_columns_far_below_the_rest(gpu, low):
+    """Half a sector's columns many orders below the others, where the block
+    rounds alone do not converge: split as rocSOLVER's Jacobi did."""
+    print("[case] split far below", low, flush=True)
+    rng = np.random.default_rng(47)
+    M = rng.standard_normal((50, 34)) * np.where(rng.permutation(34) < 17, 1.0, 10.0 ** low)
+    M /= np.linalg.norm(M)
+    out = split(gpu, one_sector(M))
+    assert out["chi"] == 17
+    assert np.max(np.abs(np.asarray(out["lam"][0]) - np.linalg.svd(M, compute_uv=False)[:17])) <= 1e-14
 
 
 def test_split_with_a_negligible_sector(gpu):
