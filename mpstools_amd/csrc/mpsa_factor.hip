@@ -817,6 +817,7 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
   if (phases & kPhApply) house_apply<C, kThreads>(X, r, false, Hv, beta, p, r, vl);
   if (!(phases & kPhOut)) return;
   // singular values (column norms of the rotated A) and their descending order
+  if (tid == 0) rotated = r;  // from here: the rank of the first zero singular value
   for (int j = wave; j < r; j += kWaves) {
     double a = 0.0;
     for (int row = lane; row < r; row += 64) {
@@ -850,6 +851,7 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
     const double sj = sig[j];
     for (int i = 0; i < r; ++i) rk += (sig[i] > sj || (sig[i] == sj && i < j)) ? 1 : 0;
     rank[j] = rk;
+    if (sj == 0.0) atomicMin(&rotated, rk);
     S[t.s_off + rk] = sj * scale;
   }
   __syncthreads();
@@ -886,80 +888,134 @@ __global__ __launch_bounds__(kThreads) void svd_jacobi_kernel(const SvdTask* __r
   }
   __syncthreads();
   // orthonormal completion of the r-side vectors of zero singular values
-  // (descending order puts them last): vectors of length r stored at
-  // base + idx * vs with stride es between elements (V^dagger rows: es = k,
-  // vs = 1; U columns: es = 1, vs = m).  The conjugate of a V^dagger row is
-  // the vector.
+  // (descending order puts them last, from rank `first` on): vectors of length
+  // r stored at base + idx * vs with stride es between elements (V^dagger rows:
+  // es = k, vs = 1; U columns: es = 1, vs = m).  The conjugate of a V^dagger
+  // row is the vector.  Each starts from a unit vector e_c and loses its
+  // components along the vectors before it, twice; c is the first index whose
+  // residual 1 - sum |u_i[c]|^2 is above 1/4, or the one of the largest
+  // residual (at least 1 / r).  All components of a pass are taken at once, so
+  // a vector costs seven barriers, where unit vectors tried one after another,
+  // component by component, cost r^2 of them: the zero sector of 160 x 160
+  // took 2.7 million (and a null space whose residuals are all below 1/4 got
+  // no vector).  60 x 60 zeros: 73.5 ms so, 0.9 ms here; a sector of nothing
+  // but zeros takes the unit vectors as they are.
+  const int first = rotated;
   const int64_t es = wide ? 1 : k, vs = wide ? m : 1;
   double* Br = wide ? Ur : Vr;
   double* Bi = wide ? Ui : Vi;
-  const double csign = wide ? 1.0 : -1.0;  // stored imaginary part = csign * vector imaginary part
-  for (int rk = 0; rk < k; ++rk) {
-    if (S[t.s_off + rk] > 0.0) continue;
-    for (int cand = 0; cand < r; ++cand) {
-      // w = e_cand, then two passes of w -= (u_i^H w) u_i over i < rk
-      for (int row = tid; row < r; row += kThreads) {
-        Br[rk * vs + row * es] = row == cand ? 1.0 : 0.0;
-        if (C) Bi[rk * vs + row * es] = 0.0;
+  if (first == 0) {
+    for (int64_t e = tid; e < (int64_t)r * r; e += kThreads) {
+      const int i = (int)(e / r), c = (int)(e % r);
+      Br[i * vs + c * es] = i == c ? 1.0 : 0.0;
+      if (C) Bi[i * vs + c * es] = 0.0;
+    }
+    __syncthreads();
+  } else if (first < k) {
+    const double csign = wide ? 1.0 : -1.0;  // stored imaginary part = csign * vector imaginary part
+    double *const wr = buf, *const wi = buf + kSvdMaxR;                     // the vector
+    double *const dr = buf + 2 * kSvdMaxR, *const di = buf + 3 * kSvdMaxR;  // its components
+    static_assert(4 * kSvdMaxR <= kCap, "the completion's vectors fit");
+    double* const rho = sig;  // residual of e_c
+    for (int c = tid; c < r; c += kThreads) {
+      double x = 1.0;
+      for (int i = 0; i < first; ++i) {
+        const double ur = Br[i * vs + c * es], ui = C ? Bi[i * vs + c * es] : 0.0;
+        x -= ur * ur + ui * ui;
+      }
+      rho[c] = x;
+    }
+    __syncthreads();
+    for (int rk = first; rk < k; ++rk) {
+      // the start
+      int c = r;
+      double top = -1.0;
+      for (int x = tid; x < r; x += kThreads)
+        if (rho[x] > 0.25 ? top < 2.0 : rho[x] > top) {
+          c = x;
+          top = rho[x] > 0.25 ? 2.0 : rho[x];
+        }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const double ot = __shfl_xor(top, o, 64);
+        const int oc = __shfl_xor(c, o, 64);
+        if (ot > top || (ot == top && oc < c)) {
+          top = ot;
+          c = oc;
+        }
+      }
+      if (lane == 0) {
+        red[wave] = top;
+        mxw[wave] = c;
       }
       __syncthreads();
-      for (int pass = 0; pass < 2; ++pass)
-        for (int i = 0; i < rk; ++i) {
-          double dr = 0.0, di = 0.0;
-          for (int row = tid; row < r; row += kThreads) {
-            const double ur = Br[i * vs + row * es], wr = Br[rk * vs + row * es];
-            dr += ur * wr;
-            if (C) {
-              const double ui = csign * Bi[i * vs + row * es], wi = csign * Bi[rk * vs + row * es];
-              dr += ui * wi;
-              di += ur * wi - ui * wr;
-            }
-          }
-          dr = wave_sum(dr);
-          if (C) di = wave_sum(di);
-          if (lane == 0) {
-            red[wave] = dr;
-            redc[wave] = di;
-          }
-          __syncthreads();
-          double Dr = 0.0, Di = 0.0;
-          for (int w = 0; w < kWaves; ++w) {
-            Dr += red[w];
-            Di += redc[w];
-          }
-          for (int row = tid; row < r; row += kThreads) {
-            const double ur = Br[i * vs + row * es];
-            const double ui = C ? csign * Bi[i * vs + row * es] : 0.0;
-            // w -= (Dr + i Di) u
-            Br[rk * vs + row * es] -= Dr * ur - Di * ui;
-            if (C) Bi[rk * vs + row * es] -= csign * (Dr * ui + Di * ur);
-          }
-          __syncthreads();
+      c = mxw[0];
+      top = red[0];
+      for (int w = 1; w < kWaves; ++w)
+        if (red[w] > top || (red[w] == top && mxw[w] < c)) {
+          top = red[w];
+          c = mxw[w];
         }
       double nn = 0.0;
-      for (int row = tid; row < r; row += kThreads) {
-        const double wr = Br[rk * vs + row * es];
-        nn += wr * wr;
-        if (C) {
-          const double wi = Bi[rk * vs + row * es];
-          nn += wi * wi;
-        }
-      }
-      nn = wave_sum(nn);
-      if (lane == 0) red[wave] = nn;
-      __syncthreads();
-      double tot = 0.0;
-      for (int w = 0; w < kWaves; ++w) tot += red[w];
-      __syncthreads();
-      if (tot > 0.25) {
-        const double inv = 1.0 / sqrt(tot);
-        for (int row = tid; row < r; row += kThreads) {
-          Br[rk * vs + row * es] *= inv;
-          if (C) Bi[rk * vs + row * es] *= inv;
+      for (int pass = 0; pass < 2; ++pass) {
+        // components u_i^H w; those of e_c are conj(u_i[c])
+        if (pass == 0) {
+          for (int i = tid; i < rk; i += kThreads) {
+            dr[i] = Br[i * vs + c * es];
+            if (C) di[i] = -csign * Bi[i * vs + c * es];
+          }
+        } else {
+          for (int i = wave; i < rk; i += kWaves) {
+            double ar = 0.0, ai = 0.0;
+            for (int row = lane; row < r; row += 64) {
+              const double ur = Br[i * vs + row * es];
+              ar += ur * wr[row];
+              if (C) {
+                const double ui = csign * Bi[i * vs + row * es];
+                ar += ui * wi[row];
+                ai += ur * wi[row] - ui * wr[row];
+              }
+            }
+            ar = wave_sum(ar);
+            if (C) ai = wave_sum(ai);
+            if (lane == 0) {
+              dr[i] = ar;
+              if (C) di[i] = ai;
+            }
+          }
         }
         __syncthreads();
-        break;
+        nn = 0.0;
+        for (int row = tid; row < r; row += kThreads) {
+          double xr = pass ? wr[row] : (row == c ? 1.0 : 0.0), xi = C && pass ? wi[row] : 0.0;
+          for (int i = 0; i < rk; ++i) {
+            const double ur = Br[i * vs + row * es];
+            xr -= dr[i] * ur;
+            if (C) {
+              const double ui = csign * Bi[i * vs + row * es];
+              xr += di[i] * ui;
+              xi -= dr[i] * ui + di[i] * ur;
+            }
+          }
+          wr[row] = xr;
+          if (C) wi[row] = xi;
+          nn += xr * xr + xi * xi;
+        }
+        __syncthreads();
       }
+      nn = wave_sum(nn);
+      if (lane == 0) redc[wave] = nn;
+      __syncthreads();
+      nn = 0.0;
+      for (int w = 0; w < kWaves; ++w) nn += redc[w];
+      const double inv = 1.0 / sqrt(nn);
+      for (int row = tid; row < r; row += kThreads) {
+        const double xr = wr[row] * inv, xi = C ? wi[row] * inv : 0.0;
+        Br[rk * vs + row * es] = xr;
+        if (C) Bi[rk * vs + row * es] = csign * xi;
+        rho[row] -= xr * xr + xi * xi;
+      }
+      __syncthreads();
     }
   }
   // FixPhase (real data): first index of the largest |V^dagger[i, c]|; flip

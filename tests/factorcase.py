@@ -133,6 +133,25 @@ class Case:
         phase(OUT)
         return self.results()
 
+    def outputs(self, svds):
+        """The SVD's outputs from given ends of the sweeps: per sector the
+        rotated A (r x r, orthogonal columns) and Q Wm (p x r)."""
+        pw = self.plane[3]
+        W = self.W.cpu().numpy()
+        for t, (A, Q) in zip(self.tasks, svds):
+            p, r = Q.shape
+            for q in range(2 if self.cplx else 1):
+                part = lambda x: np.asfortranarray(x.imag if q else x.real).reshape(-1, order="F")  # noqa: E731
+                o = q * pw + t["w_off"]
+                W[o:o + p * r] = part(Q)
+                o += 2 * p * r + r * r
+                W[o:o + r * r] = part(A)
+                W[o + r * r + r] = 1.0  # the scale, after the betas
+        self.W.copy_(self.torch.from_numpy(W))
+        f = _fn("launch_svd_phase", "iiPKNS_7SvdTaskEi" + _ARRAYS + "P12ihipStream_t")
+        self._call(f, int(self.cplx), OUT, C.c_void_p(self.dt.data_ptr()), len(self.mats), *self._arrays(), self._st())
+        return self.results()
+
     def results(self):
         """(U, S, V^dagger) per sector."""
         _, au, av, _ = self.plane
