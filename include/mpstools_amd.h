@@ -149,9 +149,11 @@ int mpsa_env_apply(mpsa_plan* plan, const double* dBL, const double* dA, const d
 int mpsa_plan_info(const mpsa_plan* plan, double* flops_alg, double* flops_ref, int64_t* n_gemm1, int64_t* n_gemm2,
                    int64_t* workspace_bytes);
 /* Algorithmic flops of the two grouped GEMM stages (one vector) and the tile
- * class each stage launches with.  FP64/FP32: 0 = 128x128, 1 = 64x64,
- * 2 = 32x32.  BF16/BF16X3: 0 = 256x128, 1 = 64x64, 2 = 128x128, 3 = 256x256,
- * 4 = 32x32. */
+ * class each stage launches with: the pinned one (set_tile_class, autotune), or
+ * else that of a single vector, where batches choose theirs by their number of
+ * vectors.  FP64/FP32: 0 = 128x128, 1 = 64x64, 2 = 32x32 per workgroup,
+ * 3 = 16x16, 4 = 32x32 per wave.  BF16/BF16X3: 0 = 256x128, 1 = 64x64,
+ * 2 = 128x128, 3 = 256x256, 4 = 32x32. */
 int mpsa_plan_stage_info(const mpsa_plan* plan, double* flops_stage1, double* flops_stage2, int* tile_class1,
                          int* tile_class2);
 /* Per-stage HIP-event timing of mpsa_heff_apply on the call's stream.  When
@@ -161,10 +163,11 @@ int mpsa_plan_set_timing(mpsa_plan* plan, int enable);
 
 /* ---- tile-class tuning (no counterpart in the reference, whose tuple loop
  * hands each product to BLAS separately) ---- */
-/* Launch stage 1 or 2 of the plan with the given tile class from now on.
- * MPSA_EINVAL if the class does not exist for the plan's precision or the
- * stage does not admit it (the 256x256 class needs unit segment scales and
- * per-operand offsets below 2^31).  Results do not depend on the class in
+/* Launch stage 1 or 2 of the plan with the given tile class from now on, for
+ * any number of vectors.  MPSA_EINVAL if the class does not exist for the
+ * plan's precision or the stage does not admit it (the 256x256 class needs unit
+ * segment scales and per-operand offsets below 2^31, the wave classes leading
+ * dimensions below 2^24).  Results do not depend on the class in
  * FP64; in reduced precision they agree within the precision's bound. */
 int mpsa_plan_set_tile_class(mpsa_plan* plan, int stage, int tile_class);
 /* Autotuner of an H_eff plan with bound environments: times every admissible

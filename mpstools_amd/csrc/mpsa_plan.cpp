@@ -140,12 +140,26 @@ static std::vector<Group> parse_mpo(const mpsa_mpo* w, int d, const char* name) 
 }
 
 // ------------------------------------------------------------------ plan
+struct Shape {
+  int prec = F64, ncls = 0;
+  double fill[kMaxTileClasses] = {}, tiles[kMaxTileClasses] = {}, steps = 0;
+  bool pipe = false, wave = false;
+};
+
 struct Stage {
   std::vector<GTask> tasks;
   std::vector<GSeg> segs;
   int tiles = 0;
   int tile_class = 0;
+  bool pinned = false;  // the class is the caller's or the tuner's, for any number of vectors
   int tr = 0;
+  Shape shape;
+  // the other classes that batches take, with the tiles of one vector; their
+  // numberings follow the tasks in d_tasks
+  struct Batch {
+    int cls, tiles;
+  };
+  std::vector<Batch> batch;
   GTask* d_tasks = nullptr;
   GSeg* d_segs = nullptr;
 };
@@ -283,64 +297,98 @@ static bool class_admissible(const std::vector<GTask>& t, const std::vector<GSeg
   return cls < 3 || fits_wave_tile(segs);
 }
 
-// The tile class of a stage without tuning, from its blocks' shapes.  A large
-// tile reads fewer operand bytes per MFMA; it is taken where it is mostly
-// full and the launch has tiles enough for 256 CUs.  Measured on one MI355X
-// (us per stage, dense bonds of dimension D unless named; tiles in brackets):
-//   FP64 128x128 / 64x64: D = 2048 stage 2 4180 [1024] / 4760, D = 1500 stage 1
-//     1970 [1440] / 2010, stage 2 3110 [576: 2.25 rounds of 256] / 2570,
-//     D = 1024 stage 2 678 [256] / 589: 128x128 from 512 tiles whose rounds
-//     of 256 are at least 80 % full;
-//   FP64 64x64 / 32x32: D = 400 stage 1 72 [490] / 92, stage 2 195 [196] / 127,
-//     D = 777 510 [676] / 583, D = 100 30 [16] / 15: 64x64 from 400 tiles;
-//   BF16X3 256x256 / 64x64: D = 2048 560 / 1610, D = 1024 stage 1 82 [160] /
-//     235, stage 2 199 [64] / 184, D = 500 stage 1 47 [40] / 29, stage 2 110
-//     [16] / 49: 256x256 from 128 tiles, the other large tiles from 512;
-//   BF16X3 64x64 / 32x32: t-V sectors of 20-120 rows, 64 vectors 430 / 846,
-//     of 1-80 rows 105 / 137, Hubbard sectors of 1-31 rows, 16 vectors 319 /
-//     254: 32x32 only where 64x64 is less than 12 % full;
-//   FP64 32x32 / 16x16 wave tile: Hubbard, 16 vectors 937 / 524, XXZ sectors of
-//     1-196 rows 43 / 50: the wave tile where 32x32 is less than 40 % full.
-static int pick_class(const std::vector<GTask>& t, const std::vector<GSeg>& segs, int prec) {
-  const bool bfp = prec == BF16 || prec == BF16X3;
-  double fill[kMaxTileClasses] = {0, 0, 0, 0, 0};
-  double tiles[kMaxTileClasses] = {0, 0, 0, 0, 0};
-  for (int cls = 0; cls < num_tile_classes(prec); ++cls) {
+// What the choice of a tile class looks at: per class the share of a tile that
+// blocks fill and the tiles of one vector, the k-steps of a 64x64 tile, and the
+// classes that the stage's strides and scales rule out.
+static Shape stage_shape(const std::vector<GTask>& t, const std::vector<GSeg>& segs, int prec) {
+  Shape s;
+  s.prec = prec;
+  s.ncls = num_tile_classes(prec);
+  for (int cls = 0; cls < s.ncls; ++cls) {
     int bm, bn;
     tile_dims(prec, cls, &bm, &bn);
-    double useful = 0, padded = 0;
+    double useful = 0, padded = 0, steps = 0;
     for (auto& x : t) {
       const double nt = (double)((x.m + bm - 1) / bm) * ((x.n + bn - 1) / bn);
       useful += (double)x.m * x.n;
       padded += nt * bm * bn;
-      tiles[cls] += nt;
+      s.tiles[cls] += nt;
+      if (cls == 1)
+        for (int j = 0; j < x.nseg; ++j) steps += nt * segs[(size_t)(x.seg0 + j)].k;
     }
-    fill[cls] = padded > 0 ? useful / padded : 1.0;
+    s.fill[cls] = padded > 0 ? useful / padded : 1.0;
+    if (cls == 1) s.steps = s.tiles[1] > 0 ? steps / s.tiles[1] : 0.0;
   }
-  if (bfp) {
-    if (fill[3] >= 0.8 && tiles[3] >= 128 && fits_pipe_tile(t, segs)) return 3;
-    if (fill[0] >= 0.8 && tiles[0] >= 512) return 0;
-    if (fill[2] >= 0.8 && tiles[2] >= 512) return 2;
-    return fill[1] < 0.12 ? 4 : 1;
-  }
-  const double rounds = std::ceil(tiles[0] / 256.0);
-  if (fill[0] >= 0.8 && tiles[0] >= 512 && tiles[0] >= 0.8 * 256.0 * rounds) return 0;
-  if (fill[1] >= 0.75 && tiles[1] >= 400) return 1;
-  return fill[2] < 0.4 && fits_wave_tile(segs) ? 3 : 2;
+  s.pipe = fits_pipe_tile(t, segs);
+  s.wave = fits_wave_tile(segs);
+  return s;
 }
 
-// Number the workgroup tiles of a stage for tile class cls, in task order
-// (tiles m-fastest inside a task).
-static void assign_tiles(Stage& s, int prec, int cls) {
+// The tile class of a launch of nvec vectors without tuning.  A large tile
+// reads fewer operand bytes per MFMA; it is taken where it is mostly full (or
+// no less full than the smallest: a block of 100 rows) and the launch, all
+// vectors together, has tiles enough for 256 CUs.  Measured on one MI355X (us
+// per stage, dense bonds of dimension D unless named; tiles in brackets):
+//   FP64 128x128 / 64x64: D = 2048 stage 2 4180 [1024] / 4760, D = 1500 stage 1
+//     1970 [1440] / 2010, stage 2 3110 [576: 2.25 rounds of 256] / 2570,
+//     D = 1024 stage 2 709 [256] / 639, two vectors 1128 [512] / 1206, D = 512
+//     stage 2, 16 vectors 1131 [1024] / 1268: 128x128 from 512 tiles whose
+//     rounds of 256 are at least 80 % full;
+//   FP32 128x128 / 64x64: D = 1024 stage 2 402 [256] / 437, D = 512 stage 1
+//     63 [256] / 67, D = 256 stage 1, two vectors 36 [128] / 22: from 256;
+//   FP64 64x64 / 32x32: D = 400 stage 1 72 [490] / 92, stage 2 195 [196] / 127,
+//     D = 777 510 [676] / 583, D = 100 30 [16] / 15, 64 vectors 84 [1024] / 111
+//     (FP32 57 / 74): 64x64 from 400 tiles;
+//   BF16X3 256x256 / 64x64: D = 2048 560 / 1610, D = 1024 stage 1 82 [160] /
+//     235, stage 2 210 [64] / 192, two vectors 222 [128] / 457, D = 256 stage 1,
+//     16 vectors 38 [256] / 67: from 128 tiles; BF16 D = 1024 stage 2 88 [64] /
+//     117, D = 512 stage 1 18 [64] / 19, stage 2 51 [16] / 36: from 64; the
+//     other large tiles from 512;
+//   BF16X3 64x64 / 32x32: t-V sectors of 20-120 rows, 64 vectors 430 / 846,
+//     of 1-80 rows 105 / 137, Hubbard sectors of 1-31 rows, 16 vectors 319 /
+//     254: 32x32 where 64x64 is less than 12 % full; and where its tiles are
+//     too few for the device, D = 256 stage 2 25 [64] / 20, D = 400 stage 2 73
+//     [196] / 80 (BF16, a whole apply: 87 / 100), which is up to 448 tiles where 32x32 is much
+//     fuller (D = 150 stage 1, two vectors 8.9 [288] / 8.0), 1280 where it is
+//     fuller still (XXZ sectors of 1-80 rows, stage 1 9.3 [398] / 7.7) and 2048
+//     with long k (stage 2, 16 vectors 53 [1600] / 39; 64 vectors 105 [6400] /
+//     131);
+//   FP64 32x32 / 16x16 wave tile: Hubbard, 16 vectors 937 / 524, XXZ sectors of
+//     1-196 rows 43 / 50: the wave tile where 32x32 is less than 40 % full.
+static int pick_class(const Shape& s, int nvec) {
+  const double* fill = s.fill;
+  auto tiles = [&](int cls) { return s.tiles[cls] * nvec; };
+  if (s.prec == BF16 || s.prec == BF16X3) {
+    if (fill[3] >= 0.8 && tiles(3) >= (s.prec == BF16 ? 64 : 128) && s.pipe) return 3;
+    if (fill[0] >= 0.8 && tiles(0) >= 512) return 0;
+    if (fill[2] >= 0.8 && tiles(2) >= 512) return 2;
+    const double gain = fill[4] / fill[1];
+    const double few = gain < 1.3 ? 192 : gain < 1.5 ? 448 : s.steps < 128 ? 1280 : 2048;
+    return fill[1] < 0.12 || tiles(1) < few ? 4 : 1;
+  }
+  auto full = [&](int cls, double bar) { return fill[cls] >= bar || fill[cls] >= 0.98 * fill[2]; };
+  const double rounds = std::ceil(tiles(0) / 256.0);
+  if (full(0, 0.8) && tiles(0) >= (s.prec == F32 ? 256 : 512) && tiles(0) >= 0.8 * 256.0 * rounds) return 0;
+  if (full(1, 0.75) && tiles(1) >= 400) return 1;
+  return fill[2] < 0.4 && s.wave ? 3 : 2;
+}
+
+// Number the workgroup tiles of a task list for tile class cls, in task order
+// (tiles m-fastest inside a task); returns their count.
+static int number_tiles(std::vector<GTask>& tasks, int prec, int cls) {
   int BM, BN;
   tile_dims(prec, cls, &BM, &BN);
   int tile = 0;
-  for (auto& t : s.tasks) {
+  for (auto& t : tasks) {
     t.tiles_m = (t.m + BM - 1) / BM;
     t.tile0 = tile;
     tile += t.tiles_m * ((t.n + BN - 1) / BN);
   }
-  s.tiles = tile;
+  return tile;
+}
+
+static void assign_tiles(Stage& s, int prec, int cls) {
+  s.tiles = number_tiles(s.tasks, prec, cls);
   s.tile_class = cls;
 }
 
@@ -372,7 +420,35 @@ static void finalize_stage(Stage& s, int prec) {
   for (size_t i : ord)
     if (s.tasks[i].m > 0 && s.tasks[i].n > 0) t2.push_back(s.tasks[i]);
   s.tasks = t2;
-  assign_tiles(s, prec, pick_class(s.tasks, s.segs, prec));
+  s.shape = stage_shape(s.tasks, s.segs, prec);
+  assign_tiles(s, prec, pick_class(s.shape, 1));
+}
+
+// The classes other than the single vector's that batches of an H_eff stage
+// take, over all numbers of vectors.
+static void finalize_batches(Stage& s, int prec) {
+  for (int n = 2; n <= 4096; n = n < 64 ? n + 1 : 2 * n) {
+    const int cls = pick_class(s.shape, n);
+    bool known = cls == s.tile_class;
+    for (auto& b : s.batch) known = known || b.cls == cls;
+    if (known) continue;
+    std::vector<GTask> t = s.tasks;
+    s.batch.push_back(Stage::Batch{cls, number_tiles(t, prec, cls)});
+  }
+}
+
+// A stage's task table for a launch of nvec vectors.
+struct StageTable {
+  const GTask* tasks;
+  int tiles, cls;
+};
+static StageTable stage_table(const Stage& s, int nvec) {
+  if (nvec > 1 && !s.pinned && !s.batch.empty()) {
+    const int cls = pick_class(s.shape, nvec);
+    for (size_t i = 0; i < s.batch.size(); ++i)
+      if (s.batch[i].cls == cls) return StageTable{s.d_tasks + (i + 1) * s.tasks.size(), s.batch[i].tiles, cls};
+  }
+  return StageTable{s.d_tasks, s.tiles, s.tile_class};
 }
 
 // A grouped GEMM assembled outside a plan (block products of the compression
@@ -982,6 +1058,10 @@ static void build_plan(mpsa_plan* P, Built& b, const Tab& Ptab, const Tab& Qtab,
   if (P->cplx) complexify(P, Ptab.total, Qtab.total, Utab.total, Ytab.total, kind);
   finalize_stage(P->s1, P->prec);
   finalize_stage(P->s2, P->prec);
+  if (kind != 2) {
+    finalize_batches(P->s1, P->prec);
+    finalize_batches(P->s2, P->prec);
+  }
   finalize_mix(P);
   P->rpL_chunks = finalize_repack(P->rpL);
   P->rpR_chunks = finalize_repack(P->rpR);
@@ -990,12 +1070,23 @@ static void build_plan(mpsa_plan* P, Built& b, const Tab& Ptab, const Tab& Qtab,
   P->planes = P->prec == BF16X3 ? 2 : 1;
 }
 
+// The tasks, numbered for the stage's class, then for those of its batches.
+static GTask* upload_tasks(const Stage& s) {
+  if (s.batch.empty()) return upload(s.tasks);
+  std::vector<GTask> all = s.tasks, t = s.tasks;
+  for (auto& b : s.batch) {
+    number_tiles(t, s.shape.prec, b.cls);
+    all.insert(all.end(), t.begin(), t.end());
+  }
+  return upload(all);
+}
+
 // Plans are built on the host only; descriptors move to the device on first use.
 static void ensure_device(mpsa_plan* P) {
   if (P->on_device) return;
-  P->s1.d_tasks = upload(P->s1.tasks);
+  P->s1.d_tasks = upload_tasks(P->s1);
   P->s1.d_segs = upload(P->s1.segs);
-  P->s2.d_tasks = upload(P->s2.tasks);
+  P->s2.d_tasks = upload_tasks(P->s2);
   P->s2.d_segs = upload(P->s2.segs);
   P->d_mix = upload(P->mix);
   P->d_terms = upload(P->terms);
@@ -1050,13 +1141,15 @@ bool plan_complex(const mpsa_plan* P) { return P && P->cplx; }
 }  // namespace mpsa
 
 // =================================================================== C ABI
-// Re-number a stage's tiles for tile class cls and refresh its device task
+// Pin a stage to tile class cls: re-number its tiles and refresh its device task
 // list (same number of tasks, so the allocation is reused).  Kernels already
 // queued on `st` read the old list, so the stream drains before the copy, and
 // the copy itself is queued on `st` ahead of every later launch.
 static void set_stage_class(mpsa_plan* P, Stage& S, int prec, int cls, hipStream_t st) {
-  if (S.tile_class == cls) return;
+  if (S.pinned && S.tile_class == cls) return;
   P->drop_graph();  // the captured launches name the old class's kernel and grid
+  S.pinned = true;
+  if (S.tile_class == cls) return;
   if (P->on_device && S.d_tasks && !S.tasks.empty()) HIPCHK(hipStreamSynchronize(st));
   assign_tiles(S, prec, cls);
   if (P->on_device && S.d_tasks && !S.tasks.empty()) {
@@ -1077,16 +1170,18 @@ static void launch_stage(mpsa_plan* P, int which, const double* dx, int64_t x_st
     pl1.a = P->Lc_elems;
     pl1.b = P->xc_per_vec;
     pl1.c = P->ws_per_vec;
-    HIPCHK(launch_gemm(P->prec, 0, P->s1.tr, P->s1.tile_class, P->s1.d_tasks, (int)P->s1.tasks.size(),
-                       P->s1.d_segs, P->s1.tiles, nvec, A1, 0, B1, P->prec == F64 ? x_stride : xcs, P->ws, wss, st,
+    const StageTable t = stage_table(P->s1, nvec);
+    HIPCHK(launch_gemm(P->prec, 0, P->s1.tr, t.cls, t.tasks, (int)P->s1.tasks.size(), P->s1.d_segs, t.tiles, nvec,
+                       A1, 0, B1, P->prec == F64 ? x_stride : xcs, P->ws, wss, st,
                        pl1));
   } else {
     const void* B2 = P->prec == F64 ? (const void*)P->dR : P->Rc;
     Planes pl2;
     pl2.a = P->ws_per_vec;
     pl2.b = P->Rc_elems;
-    HIPCHK(launch_gemm(P->prec, 1, P->s2.tr, P->s2.tile_class, P->s2.d_tasks, (int)P->s2.tasks.size(),
-                       P->s2.d_segs, P->s2.tiles, nvec, P->ws, wss, B2, 0, dy, y_stride, st, pl2));
+    const StageTable t = stage_table(P->s2, nvec);
+    HIPCHK(launch_gemm(P->prec, 1, P->s2.tr, t.cls, t.tasks, (int)P->s2.tasks.size(), P->s2.d_segs, t.tiles, nvec,
+                       P->ws, wss, B2, 0, dy, y_stride, st, pl2));
   }
 }
 

@@ -50,6 +50,7 @@ std::string g_ctx = "-";
 // every block round rotates: a sector SVD that does not converge (the
 // one-workgroup sweeps after them answer with NaN)
 bool g_rotating = false, g_swept = false;
+int g_cls[2] = {-1, -1};  // tile classes of the last two grouped GEMM launches, the latest last
 std::vector<std::string> g_msgs;
 
 void report(const std::string& m) {
@@ -133,6 +134,10 @@ extern "C" {
 long emu_violations() { return g_viol; }
 const char* emu_message(int i) { return i < (int)g_msgs.size() ? g_msgs[(size_t)i].c_str() : nullptr; }
 long emu_launches() { return g_launch; }
+void emu_gemm_classes(int* out) {
+  out[0] = g_cls[0];
+  out[1] = g_cls[1];
+}
 void emu_set_rotating(int on) { g_rotating = on != 0; }
 long emu_live_bytes() {
   long b = 0;
@@ -679,6 +684,8 @@ hipError_t launch_gemm(int prec_in, int out_kind, int tr, int tile_class, const 
                        const GSeg* segs, int tiles_per_vec, int nvec, const void* A, int64_t a_vs, const void* B,
                        int64_t b_vs, void* C, int64_t c_vs, hipStream_t st, Planes) {
   if (tiles_per_vec * nvec <= 0) return hipSuccess;
+  g_cls[0] = g_cls[1];
+  g_cls[1] = tile_class;
   int bm = 64, bn = 64;
   tile_dims(prec_in, tile_class, &bm, &bn);
   const bool TA = (tr >> 1) & 1, TB = tr & 1;

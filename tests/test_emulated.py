@@ -203,6 +203,42 @@ def test_emulated_tile_classes_agree_and_autotune_keeps_ties(lib, oracle):
     del plan
 
 
+def test_emulated_tile_class_follows_the_number_of_vectors(lib, oracle):
+    """Without tuning, a batch takes the tile that its vectors together fill the
+    device with (dense D = 64: 32x32 for one vector, 64x64 where 64 vectors make
+    1024 tiles of stage 1), with the single vector's bits; a pinned class holds
+    for any number of vectors, and the single vector's class stays its own."""
+    P = problems.build(oracle, "xxz", 14, 0, 64, 109, dense=True)
+    c, mpo, itk = P["c"], P["mpo"], P["itk"]
+    L, R, psi = P["Ls"][c - 1], P["Rs"][c + 2], P["psi"]
+    Lt, Rt, xt = native.Table.from_blocks(L), native.Table.from_blocks(R), native.Table.from_blocks(psi)
+    vt = xt.union(native.heff2_outkeys(Lt, Rt, xt, mpo[c], mpo[c + 1], itk[c], itk[c + 1]))
+    plan = native.HeffPlan(Lt, Rt, vt, vt, (mpo[c], mpo[c + 1]), (itk[c], itk[c + 1]), native.F64)
+    plan.bind_env(DevBuf(lib, Lt.pack(L)), DevBuf(lib, Rt.pack(R)))
+    x1 = vt.pack(psi)
+
+    def classes():
+        out = (C.c_int * 2)()
+        lib.emu_gemm_classes(out)
+        return tuple(out)
+
+    def apply(nvec):
+        x, y = DevBuf(lib, np.tile(x1, nvec)), DevBuf(lib, np.zeros(nvec * vt.total))
+        plan.apply(x, y, nvec, vt.total, vt.total)
+        return y.host().reshape(nvec, -1)
+
+    y1 = apply(1)[0]
+    assert classes() == (2, 2)
+    y64 = apply(64)
+    assert classes() == (1, 2)
+    assert all(np.array_equal(y, y1) for y in y64)
+    assert np.array_equal(apply(1)[0], y1) and classes() == (2, 2)
+    plan.set_tile_class(1, 2)  # its own class, pinned
+    assert all(np.array_equal(y, y1) for y in apply(64)) and classes() == (2, 2)
+    plan.set_tile_class(2, 0)
+    assert all(np.array_equal(y, y1) for y in apply(3)) and classes() == (2, 0)
+
+
 @pytest.mark.parametrize("V", [None, 0.7])
 def test_emulated_hubbard_plans_match_oracle(lib, oracle, V):
     """Plans over U(1) x U(1) packed charges and d = 4 (FermiHubbardMPO): the

@@ -59,3 +59,50 @@ def test_folded_batches(gpu, oracle, model, L, N, D, seed, dense, nvecs):
                 num = sum(float(np.sum((blocks[k] - want[k]) ** 2)) for k in want.keys())
                 den = sum(float(np.sum(want[k] ** 2)) for k in want.keys())
                 assert (num / den) ** 0.5 <= (1e-13 if prec == native.F64 else 2e-6), (prec, nvec, cls)
+
+
+@pytest.mark.parametrize("D,nvecs", [(64, (2, 64)), (100, (2, 16, 64)), (192, (3, 16)), (256, (2, 4, 16))])
+def test_untuned_batches_of_a_dense_bond(gpu, oracle, D, nvecs):
+    """The class that a batch takes by its number of vectors: the single-vector
+    apply's result bit for bit in FP64, and within the precision's bound of it
+    elsewhere (FP32 5e-6, BF16X3 2e-4, BF16 3e-2: operands rounded once, sums in
+    another order); again the same after the batches, with and without a pinned
+    class."""
+    torch = gpu
+    L = 18
+    P = problems.build(oracle, "xxz", L, 0, D, 905, dense=True)
+    c, mpo, itk = P["c"], P["mpo"], P["itk"]
+    Lt, Rt, xt = (native.Table.from_blocks(b) for b in (P["Ls"][c - 1], P["Rs"][c + 2], P["psi"]))
+    vt = xt.union(native.heff2_outkeys(Lt, Rt, xt, mpo[c], mpo[c + 1], itk[c], itk[c + 1]))
+    dL, dR = (torch.from_numpy(t.pack(b)).cuda() for t, b in ((Lt, P["Ls"][c - 1]), (Rt, P["Rs"][c + 2])))
+    rng = np.random.default_rng(D)
+    stride = vt.total + 3
+    x = torch.from_numpy(rng.standard_normal((max(nvecs), stride))).cuda()
+    ref = None
+    for prec, tol in ((native.F64, 0.0), (native.F32, 5e-6), (native.BF16X3, 2e-4), (native.BF16, 3e-2)):
+        plan = native.HeffPlan(Lt, Rt, vt, vt, (mpo[c], mpo[c + 1]), (itk[c], itk[c + 1]), prec)
+        plan.bind_env(dL, dR)
+        one = torch.full_like(x, 7.0)  # the gaps between blocks stay as they were
+        for v in range(max(nvecs)):
+            plan.apply(x[v], one[v])
+        torch.cuda.synchronize()
+        ref = one if prec == native.F64 else ref
+        own = (plan.stage_info()["tile_class1"], plan.stage_info()["tile_class2"])
+        for pin in (False, True):
+            if pin:
+                plan.set_tile_class(1, 1)
+                plan.set_tile_class(2, 1)
+            for nvec in nvecs + (1,):
+                print("[case] untuned", D, prec, nvec, pin, flush=True)
+                y = torch.full_like(x, 7.0)
+                plan.apply(x, y, nvec, stride, stride)
+                torch.cuda.synchronize()
+                for v in range(nvec):
+                    got, want = y[v, :vt.total], one[v, :vt.total]
+                    if prec == native.F64:
+                        assert torch.equal(got, want), (nvec, v)
+                    else:
+                        assert float((got - ref[v, :vt.total]).norm() / ref[v, :vt.total].norm()) <= tol, (prec, nvec)
+                assert bool((y[:, vt.total:] == 7.0).all()) and bool((y[nvec:] == 7.0).all())
+            if not pin:
+                assert (plan.stage_info()["tile_class1"], plan.stage_info()["tile_class2"]) == own
