@@ -93,11 +93,20 @@ constexpr double kDmTail = 1e-4;
 // workgroups share a sector) go to the library's batched one-sided Jacobi SVD
 // (mpsa_factor.hip), all of them in the same launches; larger ones to
 // rocSOLVER's gesvdj, one call and one wait each.  The t-V D = 512 bond (16
-// sectors of up to 160 x 160): 166 ms by gesvdj, 4.7 ms here.
+// sectors of up to 160 x 160): 166 ms by gesvdj, 4.7 ms here; one sector of
+// 64 x 64 4.7 / 1.5 ms, 512 x 512 77 / 17.5, 512 x 1024 80 / 19.4, 30 x 1024
+// 1.8 / 1.5, 2 x 4096 0.6 / 0.3.
 constexpr int64_t kOwnBlockR = 32, kOwnMaxR = kSvdBlockMaxR, kOwnMaxP = 4096;
 bool own_svd(int64_t m, int64_t n) {
   const int64_t r = std::min(m, n), p = std::max(m, n);
   return r <= kOwnMaxR && p <= (r < kOwnBlockR ? kOwnMaxP : (int64_t)kVecRowsMax);
+}
+// A long sector of the one-workgroup kernel takes its reflections through
+// memory.  One alone is gesvdj's (30 x 4096 2.8 ms against 5.0, 30 x 1536 2.1 /
+// 2.4, 24 x 4096 2.3 / 3.2; 20 x 2048 1.5 / 1.5), two together are not (30 x
+// 4096 5.4 / 4.9, 30 x 1536 3.9 / 2.4).
+bool long_sector(int64_t m, int64_t n) {
+  return std::min(m, n) > 20 && std::max(m, n) > kVecRowsMax && own_svd(m, n);
 }
 
 // one rocBLAS handle per device, created on first use
@@ -296,6 +305,11 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
     if (!cm) cm = do_trunc ? 100u : 200u;  // split :1257-1258
     const bool count_limited = (int64_t)cm < tot_S;
     auto dm_route = [&](const Sector& S) { return count_limited && std::min(S.m, S.n) >= kPrecondMin; };
+    int nlong = 0;
+    for (auto& kv : secs) nlong += long_sector(kv.second.m, kv.second.n) ? 1 : 0;
+    auto own = [&](const Sector& S) {
+      return !dm_route(S) && own_svd(S.m, S.n) && !(nlong == 1 && long_sector(S.m, S.n));
+    };
     int64_t big_ss = 0, big_mn = 0, big_s = 0;
     const bool left_bare = direction > 0;
     for (auto& kv : secs) {
@@ -332,7 +346,7 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
     int64_t w_total = 0;
     for (auto& kv : secs) {
       const Sector& S = kv.second;
-      if (S.k == 0 || dm_route(S) || !own_svd(S.m, S.n)) continue;
+      if (S.k == 0 || !own(S)) continue;
       SvdTask t{};
       t.a_off = S.off_M;
       t.u_off = S.off_U;
@@ -370,7 +384,7 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
     std::vector<std::unique_ptr<DevArr<Copy2D>>> big_dmoves;
     for (auto& kv : secs) {
       Sector& S = kv.second;
-      if (S.k == 0 || (!dm_route(S) && own_svd(S.m, S.n))) continue;
+      if (S.k == 0 || own(S)) continue;
       need_handle();
       const rocblas_int m = (rocblas_int)S.m, n = (rocblas_int)S.n, k = (rocblas_int)S.k;
       double* Ms = M.p + S.off_M;
@@ -510,7 +524,7 @@ int mpsa_split(const mpsa_blocks* psi, const double* dpsi, const uint64_t* itoke
     // NaN: a sector that the batched SVD has no factors of
     for (auto& kv : secs) {
       const Sector& S = kv.second;
-      if (dm_route(S) || !own_svd(S.m, S.n)) continue;
+      if (!own(S)) continue;
       for (int64_t i = 0; i < S.k; ++i)
         if (!std::isfinite(sv[(size_t)(S.off_S + i)])) throw SErr(MPSA_EINVAL, "split: sector SVD did not converge");
     }

@@ -50,6 +50,7 @@ std::string g_ctx = "-";
 // every block round rotates: a sector SVD that does not converge (the
 // one-workgroup sweeps after them answer with NaN)
 bool g_rotating = false, g_swept = false;
+long g_gesvdj = 0;  // rocsolver_dgesvdj calls
 int g_cls[2] = {-1, -1};  // tile classes of the last two grouped GEMM launches, the latest last
 std::vector<std::string> g_msgs;
 
@@ -134,6 +135,7 @@ extern "C" {
 long emu_violations() { return g_viol; }
 const char* emu_message(int i) { return i < (int)g_msgs.size() ? g_msgs[(size_t)i].c_str() : nullptr; }
 long emu_launches() { return g_launch; }
+long emu_gesvdj_calls() { return g_gesvdj; }
 void emu_gemm_classes(int* out) {
   out[0] = g_cls[0];
   out[1] = g_cls[1];
@@ -321,6 +323,7 @@ rocblas_status rocsolver_dgesvdj(rocblas_handle h, const rocblas_svect ls, const
                                  const double, double* residual, const rocblas_int, rocblas_int* n_sweeps,
                                  double* Sg, double* U, const rocblas_int ldu, double* V, const rocblas_int ldv,
                                  rocblas_int* info) {
+  ++g_gesvdj;
   submit(nullptr, "rocsolver_dgesvdj outputs", [=]() {
     if (check(residual, 8, "gesvdj residual")) *residual = 0.0;
     if (check(n_sweeps, sizeof(rocblas_int), "gesvdj sweeps")) *n_sweeps = 1;

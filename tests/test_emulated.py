@@ -454,6 +454,33 @@ def test_emulated_factorisations_refuse_nan(lib, oracle):
             eng.compress(0, 4)
 
 
+@pytest.mark.parametrize("shapes,calls", [([(24, 1026)], 1), ([(1200, 22)], 1), ([(24, 1026), (24, 1026)], 0),
+                                          ([(24, 1024)], 0), ([(20, 1200)], 0), ([(24, 1026), (10, 12)], 1),
+                                          ([(34, 1026)], 1)])
+def test_emulated_split_routes_of_long_sectors(lib, oracle, shapes, calls):
+    """A long sector alone among the batched SVD's is rocSOLVER's; two are not,
+    nor is one at the limits; sectors beyond the batched SVD's are either way."""
+    rng = np.random.default_rng(6)
+    psi = Blocks(2)
+    for q, (m, n) in enumerate(shapes):
+        for s1 in range(2):
+            for s2 in range(2):
+                psi[(9 * q, 9 * q, s1, s2)] = np.asfortranarray(rng.standard_normal((m // 2, n // 2)))
+    itk = native._itk([0, 0])
+    t = native.Table.from_blocks(psi)
+    lib.emu_gesvdj_calls.restype = C.c_long
+    n0 = lib.emu_gesvdj_calls()
+    h = C.c_void_p()
+    native._check(native.lib().mpsa_split(C.byref(t.s), DevBuf(lib, t.pack(psi)).p, native._ptr(itk), 2,
+                                          native._ptr(itk), 2, 1, 10 ** 6, 0, 0.0, 1, C.byref(h), C.c_void_p(0)))
+    chi = np.zeros(1, np.int32)
+    native._check(native.lib().mpsa_split_info(h, native._ptr(np.zeros(1)), native._ptr(chi),
+                                               *(native._ptr(np.zeros(1, np.int64)) for _ in range(5))))
+    native.lib().mpsa_split_destroy(h)
+    assert int(chi[0]) == sum(min(s) for s in shapes)
+    assert lib.emu_gesvdj_calls() - n0 == calls
+
+
 def test_emulated_sector_svds_that_do_not_converge(lib, oracle):
     """Block rounds that never stop rotating end at the sweep limit with the
     error of the split and of the Chebyshev engine."""

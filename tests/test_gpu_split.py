@@ -220,12 +220,12 @@ def test_split_density_route_count_limited(gpu, oracle, direction, chimax, kept)
 
 
 @pytest.mark.parametrize("dl,dr", [(1, 1), (1, 20), (15, 16), (16, 16), (17, 33), (40, 16), (16, 512), (16, 513),
-                                   (4, 2048), (4, 2049), (256, 256), (257, 256)])
+                                   (4, 2048), (4, 2049), (256, 256), (257, 256), (11, 513), (600, 12)])
 @pytest.mark.parametrize("direction", [1, 0])
 def test_split_at_the_limits_of_the_batched_svd(gpu, dl, dr, direction):
     """One dense 2 dl x 2 dr sector on either side of the lines of the sector
     SVD's dispatch (one workgroup below 32 singular values, several from 32 to
-    512 with at most 1024 rows, rocSOLVER beyond), against numpy's SVD.  Full
+    512 with at most 1024 rows, rocSOLVER beyond and for one long sector alone), against numpy's SVD.  Full
     rank with singular values 1 .. 2^-k, k < 8, so every vector is determined:
     bars as in _cmp_lambda, the rebuilt state and the isometry within 1e-12
     (n eps is below 1e-12 up to n = 4096)."""
