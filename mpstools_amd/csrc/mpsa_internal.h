@@ -68,8 +68,27 @@ struct Planes {
 // a_vs/b_vs/c_vs are per-vector strides (elements) for batched launches.
 hipError_t launch_gemm(int prec_in, int out_kind, int tr, int tile_class, const GTask* tasks, int ntasks,
                        const GSeg* segs, int tiles_per_vec, int nvec, const void* A, int64_t a_vs, const void* B,
-                       int64_t b_vs, void* C, int64_t c_vs, hipStream_t st, Planes planes = Planes());
-// out_kind: 0 = same type as the input precision, 1 = double
+                       int64_t b_vs, void* C, int64_t c_vs, hipStream_t st, Planes planes = Planes(),
+                       int64_t max_dim = 0);
+// out_kind: 0 = same type as the input precision, 1 = double; max_dim: the
+// tasks' largest m or n where a batched launch may fold its vectors, 0: never
+//
+// Which operand a batched FP64/FP32 launch folds over its vectors (tile_pos in
+// mpsa_kernels.hip): the columns where all vectors share A (T = L x), the rows
+// where they share B (y = T R^T); the forms of an H_eff apply, the only batched
+// launches.  At most 4096 vectors (fold_pos), and the folded dimension rounded
+// up to a tile of 128 below 2^31.
+constexpr int fold_of(int tr, int64_t nvec, int64_t a_vs, int64_t b_vs, int64_t max_dim) {
+  if (nvec <= 1 || nvec > 4096 || max_dim <= 0 || max_dim * nvec >= (int64_t(1) << 31) - 128) return 0;
+  if (tr == 0 && a_vs == 0 && b_vs != 0) return 1;
+  if (tr == 1 && b_vs == 0 && a_vs != 0) return 2;
+  return 0;
+}
+static_assert(fold_of(0, 4096, 0, 1, 524287) == 1 && fold_of(1, 4096, 1, 0, 524287) == 2, "up to 2^31");
+static_assert(fold_of(0, 4096, 0, 1, 524288) == 0 && fold_of(1, 4, 1, 0, 1 << 29) == 0, "2^31 and beyond: per vector");
+static_assert(fold_of(0, 4097, 0, 1, 8) == 0 && fold_of(0, 1, 0, 1, 8) == 0 && fold_of(2, 16, 0, 1, 8) == 0 &&
+                  fold_of(0, 16, 0, 1, 0) == 0,
+              "other launches: per vector");
 hipError_t launch_mix(int prec, const MixTask* tasks, int ntasks, const MixTerm* terms, int chunks_per_vec, int nvec,
                       const void* src, void* dst, int64_t vs, hipStream_t st, int64_t plane = 0);
 hipError_t launch_convert(int prec, const double* src, void* dst, int64_t n, hipStream_t st);

@@ -2549,27 +2549,16 @@ int gemm_max_grid(int prec_in, int tile_class) {
   return num_cu() * 2;
 }
 
-// Which operand a batched launch folds over its vectors (see tile_pos): the
-// columns where all vectors share A (T = L x), the rows where they share B
-// (y = T R^T); the forms of an H_eff apply, the only batched launches.
-// At most 4096 vectors: a folded row or column number stays below 2^31.
-static int fold_of(int tr, int nvec, int64_t a_vs, int64_t b_vs) {
-  if (nvec <= 1 || nvec > 4096) return 0;
-  if (tr == 0 && a_vs == 0 && b_vs != 0) return 1;
-  if (tr == 1 && b_vs == 0 && a_vs != 0) return 2;
-  return 0;
-}
-
 template <typename T, typename TOut, int WT>
-static hipError_t runwave(int tr, const GTask* tasks, int ntasks, const GSeg* segs, int tpv, int nvec, const void* A,
-                          int64_t a_vs, const void* B, int64_t b_vs, void* C, int64_t c_vs, hipStream_t st) {
+static hipError_t runwave(int fold, int tr, const GTask* tasks, int ntasks, const GSeg* segs, int tpv, int nvec,
+                          const void* A, int64_t a_vs, const void* B, int64_t b_vs, void* C, int64_t c_vs,
+                          hipStream_t st) {
   const int total = tpv * nvec;
   if (total <= 0) return hipSuccess;
   int grid = num_cu() * (sizeof(T) == 4 ? (WT == 16 ? 8 : 5) : (WT == 16 ? 6 : 4));  // what the registers allow
   const int need = (total + 3) / 4;
   if (grid > need) grid = need;
   if (grid >= 8) grid &= ~7;
-  const int fold = fold_of(tr, nvec, a_vs, b_vs);
   const T* a = (const T*)A;
   const T* b = (const T*)B;
   TOut* c = (TOut*)C;
@@ -2583,11 +2572,11 @@ static hipError_t runwave(int tr, const GTask* tasks, int ntasks, const GSeg* se
 }
 
 template <typename T, typename TOut, int BM, int BN>
-static hipError_t run16(int tr, const GTask* tasks, int ntasks, const GSeg* segs, int tpv, int nvec, const void* A,
-                        int64_t a_vs, const void* B, int64_t b_vs, void* C, int64_t c_vs, hipStream_t st) {
+static hipError_t run16(int fold, int tr, const GTask* tasks, int ntasks, const GSeg* segs, int tpv, int nvec,
+                        const void* A, int64_t a_vs, const void* B, int64_t b_vs, void* C, int64_t c_vs,
+                        hipStream_t st) {
   const int total = tpv * nvec;
   if (total <= 0) return hipSuccess;
-  const int fold = fold_of(tr, nvec, a_vs, b_vs);
   // persistent workgroups per CU: the small tiles run several per CU so that
   // the short-k tiles of small sectors overlap their load latency; 128x128
   // keeps two (its registers and two LDS buffers allow no more)
@@ -2649,18 +2638,24 @@ static hipError_t runbf(const GTask* tasks, int ntasks, const GSeg* segs, int tp
 
 hipError_t launch_gemm(int prec_in, int out_kind, int tr, int tile_class, const GTask* tasks, int ntasks,
                        const GSeg* segs, int tiles_per_vec, int nvec, const void* A, int64_t a_vs, const void* B,
-                       int64_t b_vs, void* C, int64_t c_vs, hipStream_t st, Planes planes) {
-#define MPSA_RUN16(T_, TO_)                                                                                    \
-  do {                                                                                                       \
-    if (tile_class == 0)                                                                                     \
-      return run16<T_, TO_, 128, 128>(tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs, st); \
-    if (tile_class == 2)                                                                                     \
-      return run16<T_, TO_, 32, 32>(tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs, st);   \
-    if (tile_class == 3)                                                                                     \
-      return runwave<T_, TO_, 16>(tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs, st);     \
-    if (tile_class == 4)                                                                                     \
-      return runwave<T_, TO_, 32>(tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs, st);     \
-    return run16<T_, TO_, 64, 64>(tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs, st);     \
+                       int64_t b_vs, void* C, int64_t c_vs, hipStream_t st, Planes planes, int64_t max_dim) {
+  const int fold = fold_of(tr, nvec, a_vs, b_vs, max_dim);
+#define MPSA_RUN16(T_, TO_)                                                                                        \
+  do {                                                                                                             \
+    if (tile_class == 0)                                                                                           \
+      return run16<T_, TO_, 128, 128>(fold, tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs,\
+                                      st);                                                                         \
+    if (tile_class == 2)                                                                                           \
+      return run16<T_, TO_, 32, 32>(fold, tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs, \
+                                    st);                                                                           \
+    if (tile_class == 3)                                                                                           \
+      return runwave<T_, TO_, 16>(fold, tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs,   \
+                                  st);                                                                             \
+    if (tile_class == 4)                                                                                           \
+      return runwave<T_, TO_, 32>(fold, tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs,   \
+                                  st);                                                                             \
+    return run16<T_, TO_, 64, 64>(fold, tr, tasks, ntasks, segs, tiles_per_vec, nvec, A, a_vs, B, b_vs, C, c_vs,   \
+                                  st);                                                                             \
   } while (0)
   if (prec_in == F64) MPSA_RUN16(double, double);
   if (prec_in == F32) {

@@ -143,6 +143,7 @@ static std::vector<Group> parse_mpo(const mpsa_mpo* w, int d, const char* name) 
 struct Shape {
   int prec = F64, ncls = 0;
   double fill[kMaxTileClasses] = {}, tiles[kMaxTileClasses] = {}, steps = 0;
+  int64_t max_dim = 0;  // largest rows or columns of a block
   bool pipe = false, wave = false;
 };
 
@@ -319,6 +320,7 @@ static Shape stage_shape(const std::vector<GTask>& t, const std::vector<GSeg>& s
     s.fill[cls] = padded > 0 ? useful / padded : 1.0;
     if (cls == 1) s.steps = s.tiles[1] > 0 ? steps / s.tiles[1] : 0.0;
   }
+  for (auto& x : t) s.max_dim = std::max<int64_t>(s.max_dim, std::max(x.m, x.n));
   s.pipe = fits_pipe_tile(t, segs);
   s.wave = fits_wave_tile(segs);
   return s;
@@ -1172,8 +1174,7 @@ static void launch_stage(mpsa_plan* P, int which, const double* dx, int64_t x_st
     pl1.c = P->ws_per_vec;
     const StageTable t = stage_table(P->s1, nvec);
     HIPCHK(launch_gemm(P->prec, 0, P->s1.tr, t.cls, t.tasks, (int)P->s1.tasks.size(), P->s1.d_segs, t.tiles, nvec,
-                       A1, 0, B1, P->prec == F64 ? x_stride : xcs, P->ws, wss, st,
-                       pl1));
+                       A1, 0, B1, P->prec == F64 ? x_stride : xcs, P->ws, wss, st, pl1, P->s1.shape.max_dim));
   } else {
     const void* B2 = P->prec == F64 ? (const void*)P->dR : P->Rc;
     Planes pl2;
@@ -1181,7 +1182,7 @@ static void launch_stage(mpsa_plan* P, int which, const double* dx, int64_t x_st
     pl2.b = P->Rc_elems;
     const StageTable t = stage_table(P->s2, nvec);
     HIPCHK(launch_gemm(P->prec, 1, P->s2.tr, t.cls, t.tasks, (int)P->s2.tasks.size(), P->s2.d_segs, t.tiles, nvec,
-                       P->ws, wss, B2, 0, dy, y_stride, st, pl2));
+                       P->ws, wss, B2, 0, dy, y_stride, st, pl2, P->s2.shape.max_dim));
   }
 }
 

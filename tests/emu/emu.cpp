@@ -685,7 +685,7 @@ static void gemm16(int BM, int BN, bool TA, bool TB, const GTask* tasks, int nta
 
 hipError_t launch_gemm(int prec_in, int out_kind, int tr, int tile_class, const GTask* tasks, int ntasks,
                        const GSeg* segs, int tiles_per_vec, int nvec, const void* A, int64_t a_vs, const void* B,
-                       int64_t b_vs, void* C, int64_t c_vs, hipStream_t st, Planes) {
+                       int64_t b_vs, void* C, int64_t c_vs, hipStream_t st, Planes, int64_t) {
   if (tiles_per_vec * nvec <= 0) return hipSuccess;
   g_cls[0] = g_cls[1];
   g_cls[1] = tile_class;
