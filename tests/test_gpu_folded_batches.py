@@ -10,6 +10,7 @@ sums of the same length)."""
 import numpy as np
 import pytest
 
+import complexcase as cc
 import plan_interp
 import problems
 from mpstools_amd import native
@@ -59,6 +60,44 @@ def test_folded_batches(gpu, oracle, model, L, N, D, seed, dense, nvecs):
                 num = sum(float(np.sum((blocks[k] - want[k]) ** 2)) for k in want.keys())
                 den = sum(float(np.sum(want[k] ** 2)) for k in want.keys())
                 assert (num / den) ** 0.5 <= (1e-13 if prec == native.F64 else 2e-6), (prec, nvec, cls)
+
+
+@pytest.mark.parametrize("model,L,N,D,seed,dense", [("xxz", 12, 6, 40, 911, False), ("hubbard", 8, 8, 60, 912, False),
+                                                    ("xxz", 14, 0, 37, 913, True)])
+@pytest.mark.parametrize("sites,cplx", [(1, False), (1, True), (2, True)])
+def test_folded_one_site_and_complex_batches(gpu, oracle, model, L, N, D, seed, dense, sites, cplx):
+    """One-site and complex (planar: blocks of real and imaginary parts, with
+    signs) plans at every FP64/FP32 tile class: batches equal the single-vector
+    applies bit for bit, and write nothing between the vectors."""
+    torch = gpu
+    P = problems.build(oracle, model, L, N, D, seed, dense=dense)
+    c, mpo, itk = P["c"], P["mpo"], P["itk"]
+    Lb = P["Ls"][c - 1]
+    Rb, xb = (P["Rs"][c + 2], P["psi"]) if sites == 2 else (P["Rs"][c + 1], P["mps"][c])
+    if cplx:
+        Lb, Rb, xb = (cc.with_imag(b, seed + i) for i, b in enumerate((Lb, Rb, xb)))
+    Lt, Rt, xt = (native.Table.from_blocks(b) for b in (Lb, Rb, xb))
+    W, ik = ((mpo[c], mpo[c + 1]), (itk[c], itk[c + 1])) if sites == 2 else (mpo[c], itk[c])
+    keys = native.heff2_outkeys(Lt, Rt, xt, *W, *ik) if sites == 2 else native.heff1_outkeys(Lt, Rt, xt, W, ik)
+    vt = xt.union(keys)
+    dL, dR = (torch.from_numpy(t.pack(b)).cuda() for t, b in ((Lt, Lb), (Rt, Rb)))
+    rng = np.random.default_rng(seed)
+    stride = vt.length + 5
+    x = torch.from_numpy(rng.standard_normal((17, stride))).cuda()
+    for prec in (native.F64,) if cplx else (native.F64, native.F32):
+        plan = native.HeffPlan(Lt, Rt, vt, vt, W, ik, prec)
+        plan.bind_env(dL, dR)
+        for cls in range(5):
+            plan.set_tile_class(1, cls)
+            plan.set_tile_class(2, cls)
+            for nvec in (3, 17):
+                print("[case]", model, sites, cplx, prec, cls, nvec, flush=True)
+                y, one = torch.full_like(x, 7.0), torch.full_like(x, 7.0)
+                plan.apply(x, y, nvec, stride, stride)
+                for v in range(nvec):
+                    plan.apply(x[v], one[v])
+                torch.cuda.synchronize()
+                assert torch.equal(y, one)
 
 
 @pytest.mark.parametrize("D,nvecs", [(64, (2, 64)), (100, (2, 16, 64)), (192, (3, 16)), (256, (2, 4, 16))])

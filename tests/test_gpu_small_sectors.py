@@ -1,8 +1,9 @@
-"""Small sector factorisations (held in LDS) against numpy, at the edges of
-their range: one row or column, 31 / 32 singular values (one workgroup's SVD
-below 32), wide and tall, a zero matrix, a rank-deficient one, and sectors just
-too large for LDS.  Driven through the split of a one-sector two-site state
-(the real SVD) and the orthonormalisation of a complex MPS (QR and SVD)."""
+"""Small sector factorisations against numpy: two rows or columns, 30 / 32
+singular values (one workgroup's SVD below 32), wide and tall, rank-deficient
+ones, and long ones beyond one workgroup's LDS.  Driven through the split of a
+one-sector two-site state (the real SVD) and the orthonormalisation of a complex
+MPS (QR).  The routes' exact limits are in test_gpu_sector_limits.py, zero
+sectors in test_gpu_zero_sectors.py."""
 import numpy as np
 import pytest
 
@@ -17,8 +18,8 @@ pytestmark = pytest.mark.gpu
                                         (250, 15, None), (15, 260, None), (200, 15, None), (15, 10, 6), (8, 8, 1)])
 def test_small_real_svd(gpu, dl, dr, rank):
     """Sum of singular triplets = the state within 1e-13 relative (k <= 31 terms
-    of rounding eps each), singular values within 1e-14 of the largest, kept
-    count = the rank (values above 1e-15 of a unit-norm state)."""
+    of rounding eps each), singular values within 1e-14 of the unit norm; values
+    beyond the rank, where the SVD keeps any, at 16 eps."""
     torch = gpu
     print("[case] small svd", 2 * dl, 2 * dr, rank, flush=True)
     rng = np.random.default_rng(77 * dl + dr)
