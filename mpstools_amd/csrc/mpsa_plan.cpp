@@ -350,11 +350,12 @@ static Shape stage_shape(const std::vector<GTask>& t, const std::vector<GSeg>& s
 //     of 1-80 rows 105 / 137, Hubbard sectors of 1-31 rows, 16 vectors 319 /
 //     254: 32x32 where 64x64 is less than 12 % full; and where its tiles are
 //     too few for the device, D = 256 stage 2 25 [64] / 20, D = 400 stage 2 73
-//     [196] / 80 (BF16, a whole apply: 87 / 100), which is up to 448 tiles where 32x32 is much
-//     fuller (D = 150 stage 1, two vectors 8.9 [288] / 8.0), 1280 where it is
-//     fuller still (XXZ sectors of 1-80 rows, stage 1 9.3 [398] / 7.7) and 2048
-//     with long k (stage 2, 16 vectors 53 [1600] / 39; 64 vectors 105 [6400] /
-//     131);
+//     [196] / 80: up to 192 tiles, 224 where 32x32 is much fuller (t-V sectors
+//     of 1-160 rows, stage 2 21 [210] / 18; XXZ of 1-196, a whole apply 48 [256]
+//     / 51), 448 where it is fuller still (XXZ of 1-80 rows, stage 1 9.3 [398] /
+//     7.7; t-V of 1-110, two vectors, a whole apply 36 [920] / 40) and 2048 with
+//     long k (XXZ of 1-80, stage 2, 16 vectors 53 [1600] / 39; 64 vectors 105
+//     [6400] / 131);
 //   FP64 32x32 / 16x16 wave tile: Hubbard, 16 vectors 937 / 524, XXZ sectors of
 //     1-196 rows 43 / 50: the wave tile where 32x32 is less than 40 % full.
 static int pick_class(const Shape& s, int nvec) {
@@ -365,7 +366,7 @@ static int pick_class(const Shape& s, int nvec) {
     if (fill[0] >= 0.8 && tiles(0) >= 512) return 0;
     if (fill[2] >= 0.8 && tiles(2) >= 512) return 2;
     const double gain = fill[4] / fill[1];
-    const double few = gain < 1.3 ? 192 : gain < 1.5 ? 448 : s.steps < 128 ? 1280 : 2048;
+    const double few = gain < 1.3 ? 192 : gain < 1.5 ? 224 : s.steps < 128 ? 448 : 2048;
     return fill[1] < 0.12 || tiles(1) < few ? 4 : 1;
   }
   auto full = [&](int cls, double bar) { return fill[cls] >= bar || fill[cls] >= 0.98 * fill[2]; };
