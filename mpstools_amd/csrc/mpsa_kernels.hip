@@ -245,8 +245,11 @@ __device__ __forceinline__ TilePos<FOLD> tile_pos(const GTask* __restrict__ task
 // tile.  A and B slabs of BK k-steps go through two LDS buffers (k-major), so
 // a slab costs one barrier; the next slab's global loads are issued into
 // registers before the MFMAs of the current one.  Row pitch BM + 4: the four
-// k-groups of a fragment read and the transposing writes both fall on distinct
-// banks.  A thread keeps a pointer to each of its rows for a segment; k is
+// k-groups of a fragment read and the writes of an operand with contiguous rows
+// fall on distinct banks; the transposing writes of one with contiguous k do
+// not (FP64 32x32, t-V D = 512, 64 vectors: no conflicts counted in stage 2,
+// 2.2 cycles per LDS instruction in stage 1, with LDS waits 1.3 % of the wave
+// cycles).  A thread keeps a pointer to each of its rows for a segment; k is
 // clamped to the segment and masked on its last slab, and rows past the block
 // are clamped to its last row (their results are never stored).
 // k order (all FP64/FP32 kernels of this file, so that results do not depend
