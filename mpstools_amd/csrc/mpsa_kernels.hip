@@ -2559,6 +2559,13 @@ static hipError_t runwave(int fold, int tr, const GTask* tasks, int ntasks, cons
   const int total = tpv * nvec;
   if (total <= 0) return hipSuccess;
   int grid = num_cu() * (sizeof(T) == 4 ? (WT == 16 ? 8 : 5) : (WT == 16 ? 6 : 4));  // what the registers allow
+  // Where every vector's tile has a wave of its own, folding leaves the slots of
+  // a task but its first few empty, and with nvec a multiple of 16 the full ones
+  // on every fourth workgroup or fewer, so on a part of the CUs (us per apply,
+  // folded / per vector: t-V D = 128, 16 vectors 22.5 / 20.5, XXZ D = 48, 32
+  // vectors 17.4 / 15.9; but XXZ D = 48, 12 vectors 13.3 / 15.0, Hubbard D = 32,
+  // 8 vectors 26.2 / 27.7; beyond one round, t-V D = 350, 64 vectors 191 / 197).
+  if (WT == 16 && nvec % 16 == 0 && total <= 4 * grid) fold = 0;
   const int need = (total + 3) / 4;
   if (grid > need) grid = need;
   if (grid >= 8) grid &= ~7;
